@@ -100,28 +100,28 @@ __global__ void __launch_bounds__(256) zero_bhd_kernel(char* __restrict__ p, Vie
     *reinterpret_cast<float*>(q) = 0.0f;
 }
 
-int scan_launch_fwd(bool bf16, const FwdArgs& a, ScanCfg cfg, int grid, bool vec, int gm,
+int scan_launch_fwd(bool bf16, const FwdArgs& a, ScanCfg cfg, int grid, bool vec, int gm, int rm,
                     hipStream_t st) {
-  return bf16 ? scan_fwd_launch_bf16(a, cfg, grid, vec, gm, st)
-              : scan_fwd_launch_f32(a, cfg, grid, vec, gm, st);
+  return bf16 ? scan_fwd_launch_bf16(a, cfg, grid, vec, gm, rm, st)
+              : scan_fwd_launch_f32(a, cfg, grid, vec, gm, rm, st);
 }
 
 int scan_launch_fwd_chain(bool bf16, const FwdArgs& a, const ChainArgs& ch, ScanCfg cfg, int gm,
-                          hipStream_t st) {
-  return bf16 ? scan_fwd_chain_launch_bf16(a, ch, cfg, gm, st)
-              : scan_fwd_chain_launch_f32(a, ch, cfg, gm, st);
+                          int rm, hipStream_t st) {
+  return bf16 ? scan_fwd_chain_launch_bf16(a, ch, cfg, gm, rm, st)
+              : scan_fwd_chain_launch_f32(a, ch, cfg, gm, rm, st);
 }
 
 int scan_launch_bwd(bool bf16, const BwdArgs& a, ScanCfg cfg, int grid, bool vec, int gm,
-                    bool lb, hipStream_t st) {
-  return bf16 ? scan_bwd_launch_bf16(a, cfg, grid, vec, gm, lb, st)
-              : scan_bwd_launch_f32(a, cfg, grid, vec, gm, lb, st);
+                    bool lb, int rm, hipStream_t st) {
+  return bf16 ? scan_bwd_launch_bf16(a, cfg, grid, vec, gm, lb, rm, st)
+              : scan_bwd_launch_f32(a, cfg, grid, vec, gm, lb, rm, st);
 }
 
-int scan_launch_bwd_chain(bool bf16, const BwdArgs& a, ScanCfg cfg, int grid, int gm,
+int scan_launch_bwd_chain(bool bf16, const BwdArgs& a, ScanCfg cfg, int grid, int gm, int rm,
                           hipStream_t st) {
-  return bf16 ? scan_bwd_chain_launch_bf16(a, cfg, grid, gm, st)
-              : scan_bwd_chain_launch_f32(a, cfg, grid, gm, st);
+  return bf16 ? scan_bwd_chain_launch_bf16(a, cfg, grid, gm, rm, st)
+              : scan_bwd_chain_launch_f32(a, cfg, grid, gm, rm, st);
 }
 
 int scan_launch_lb_fold(bool bf16, const BwdArgs& a, hipStream_t st) {
@@ -293,6 +293,30 @@ inline bool vec_ok(const void* p, const int64_t* s, int nd_outer, int V) {
   for (int i = 0; i < nd_outer; ++i)
     if (s[i] % V != 0) return false;
   return true;
+}
+
+// How the scan kernels read a values view (and write its gradient): a
+// time-contiguous view -- a (B, F, T) projection seen as (B, T, F), what the
+// filters' reference dataflow hands the scan -- goes through the row modes,
+// which need one gate per lane, whole vectors of channels, a head that fills 4
+// to 32 channel lanes and at least one quad of steps (T >= 4).  ROWS_EVEN:
+// rows of whole quads that start on a dword; ROWS_ANY: any other T or
+// alignment.  Element by element -- the only other way to read such a view --
+// measured slower everywhere (MI355X kernel times, element / row modes):
+//   bf16, B = 16, T = 1024, 18 heads of 128, one gate (ROWS_EVEN): forward
+//     103.2 / 36.6 us (4.1 TB/s), backward 365 / 88 us (2.6 TB/s);
+//   bf16, B = 5, T = 1501, 16 heads of 64 (ROWS_ANY): forward 49.9 / 26.2 us,
+//     backward 136 us in time chunks / 31.3 us chained;
+//   fp32, B = 8, T = 1024, 18 heads of 128 (ROWS_EVEN): forward 55.1 / 32.3 us,
+//     backward 225 us in time chunks / 92 us chained.
+int rows_mode(int dtype, const void* p, const int64_t* s, int T, int D, int r) {
+  const int V = dtype == LTV_DTYPE_BF16 ? 8 : 4;
+  if (s[2] != 1 || T < 4 || r % V != 0) return ROWS_NONE;  // (r % V == 0: so is D)
+  const int cl = next_pow2(D / V);
+  if (cl < 4 || cl > 32) return ROWS_NONE;
+  bool even = T % 4 == 0 && (reinterpret_cast<uintptr_t>(p) & 3u) == 0;
+  if (dtype == LTV_DTYPE_BF16) even = even && s[0] % 2 == 0 && s[1] % 2 == 0 && s[3] % 2 == 0;
+  return even ? ROWS_EVEN : ROWS_ANY;
 }
 
 // Launch-shape overrides, read once: LTV_SCAN_FWD_CFG="CL,L,NW" (CL = channel
@@ -580,8 +604,8 @@ ChainPlan chain_plan(int dtype, int B, int T, int H, int Da, int r) {
 
 // Forward launch over B * H * nwin windows x channel slabs (a.P/Q/K/nwin, and
 // a.wst / a.kw for the warm-up mode, already set): gate mode and launch shape.
-int launch_forward(int dtype, FwdArgs& a, bool vec, const HostView4& lg, int B, int T, int NH,
-                   int NKVH, int Da, int r, int use_sigmoid, hipStream_t st) {
+int launch_forward(int dtype, FwdArgs& a, bool vec, int rm, const HostView4& lg, int B, int T,
+                   int NH, int NKVH, int Da, int r, int use_sigmoid, hipStream_t st) {
   const int H = NH + 2 * NKVH;
   const int D = Da * r;
   const int V = dtype == LTV_DTYPE_BF16 ? 8 : 4;
@@ -604,14 +628,14 @@ int launch_forward(int dtype, FwdArgs& a, bool vec, const HostView4& lg, int B, 
   const int fcl = cl_full < 8 ? cl_full : 8;
   const int nslab0 = (D + fcl * V - 1) / (fcl * V);
   const bool few = (int64_t)B * H * a.nwin * nslab0 < 1024;
-  ScanCfg cfg{fcl, fcl == 8 && vec && !few ? 2 : 4, 4};
+  ScanCfg cfg{fcl, fcl == 8 && vec && !few && rm == ROWS_NONE ? 2 : 4, 4};
   const ScanTuning& tu = tuning();
-  if (vec && tu.fwd_cl > 0) cfg = ScanCfg{tu.fwd_cl < cl_full ? tu.fwd_cl : cl_full, tu.fwd_l, tu.fwd_nw};
+  if (vec && rm == ROWS_NONE && tu.fwd_cl > 0) cfg = ScanCfg{tu.fwd_cl < cl_full ? tu.fwd_cl : cl_full, tu.fwd_l, tu.fwd_nw};
   const int nslab = (D + cfg.CL * V - 1) / (cfg.CL * V);
   a.sh = ScanShape{B, T, NH, NKVH, Da, r, D, H, nslab, use_sigmoid};
   const int64_t grid = (int64_t)B * H * a.nwin * nslab;
   LTV_REQUIRE(grid < (1ll << 31), LTV_ERR_UNSUPPORTED, "grid too large");
-  return scan_launch_fwd(dtype == LTV_DTYPE_BF16, a, cfg, (int)grid, vec, gm, st);
+  return scan_launch_fwd(dtype == LTV_DTYPE_BF16, a, cfg, (int)grid, vec, gm, rm, st);
 }
 
 // The inits' dtype: the values' own, or fp32 with bf16 values (the parameter
@@ -663,7 +687,7 @@ int scan_forward_impl(int dtype, const HostView4& u, const HostView4& lg, const 
   if ((rc = check_tile_offsets("values", u.s, D, E)) || (rc = check_tile_offsets("logits", lg.s, D, E)) ||
       (rc = check_tile_offsets("inits", init.s, D, init_f32 ? 4 : E)))
     return rc;
-  bool vec = (D % V == 0) && vec_ok(u.p, u.s, 3, V) && vec_ok(init.p, init.s, 3, V);
+  bool vec = (D % V == 0) && vec_ok(init.p, init.s, 3, V);
   for (int i = 0; i < 3; ++i) {
     a.out.p[i] = outp[i];
     for (int k = 0; k < 4; ++k) a.out.s[i][k] = outs[i][k];
@@ -673,6 +697,12 @@ int scan_forward_impl(int dtype, const HostView4& u, const HostView4& lg, const 
       if ((rc = check_tile_offsets("outputs", outs[i], D, E))) return rc;
       vec = vec && vec_ok(outp[i], outs[i], 3, V);
     }
+  }
+  // values in 16-byte vectors too, or in time-contiguous rows
+  int rm = ROWS_NONE;
+  if (vec && !vec_ok(u.p, u.s, 3, V)) {
+    if (a.nwin == 1) rm = rows_mode(dtype, u.p, u.s, T, D, r);
+    vec = rm != ROWS_NONE;
   }
   if (a.nwin > 1 && (tuning().lb_short && lb_short_ok(V, r, Q, K))) {
     a.sh = ScanShape{B, T, NH, NKVH, Da, r, D, H, 1, use_sigmoid};
@@ -695,7 +725,10 @@ int scan_forward_impl(int dtype, const HostView4& u, const HostView4& lg, const 
   if (a.nwin == 1 && chain_ws != nullptr) {
     const ChainPlan pl = chain_plan(dtype, B, T, H, Da, r);
     const bool lg_ok = pl.gm == GATE_LANE || (pl.gm == GATE_CHANVEC && chanvec_ok(r, D, V, lg));
-    if (pl.cfg.CL > 0 && vec && lg_ok) {
+    // the row modes are built for the default chained shape
+    const bool rows_ok = rm == ROWS_NONE || (pl.gm == GATE_LANE && pl.cfg.CL == 8 &&
+                                             pl.cfg.L == 8 && pl.cfg.NW == 8);
+    if (pl.cfg.CL > 0 && vec && lg_ok && rows_ok) {
       LTV_REQUIRE(chain_ws_bytes >= pl.bytes, LTV_ERR_WORKSPACE,
                   "chained scan workspace too small: %zu bytes, need %zu", chain_ws_bytes,
                   pl.bytes);
@@ -711,10 +744,10 @@ int scan_forward_impl(int dtype, const HostView4& u, const HostView4& lg, const 
       ch.nseq = (int)pl.nseq;
       ch.nchunk = pl.nchunk;
       ch.ctl = chain_ctl(st);
-      return scan_launch_fwd_chain(dtype == LTV_DTYPE_BF16, a, ch, pl.cfg, pl.gm, st);
+      return scan_launch_fwd_chain(dtype == LTV_DTYPE_BF16, a, ch, pl.cfg, pl.gm, rm, st);
     }
   }
-  return launch_forward(dtype, a, vec, lg, B, T, NH, NKVH, Da, r, use_sigmoid, st);
+  return launch_forward(dtype, a, vec, rm, lg, B, T, NH, NKVH, Da, r, use_sigmoid, st);
 }
 
 // Upper bound on the backward's time chunks per (b, h).  With at least 256
@@ -925,8 +958,7 @@ int scan_backward_impl(int dtype, const HostView4& u, const HostView4& lg, const
       (rc = check_tile_offsets("grad logits", dlg.s, D, E)) ||
       (rc = check_tile_offsets("inits", init.s, D, EI)))
     return rc;
-  bool vec = (D % V == 0) && vec_ok(u.p, u.s, 3, V) && vec_ok(init.p, init.s, 3, V) &&
-             vec_ok(du.p, du.s, 3, V) && vec_ok(dinit.p, dinit.s, 3, V);
+  bool vec = (D % V == 0) && vec_ok(init.p, init.s, 3, V) && vec_ok(dinit.p, dinit.s, 3, V);
   for (int i = 0; i < 3; ++i) {
     a.h.p[i] = const_cast<void*>(hp[i]);
     a.gy.p[i] = const_cast<void*>(gp[i]);
@@ -942,6 +974,17 @@ int scan_backward_impl(int dtype, const HostView4& u, const HostView4& lg, const
         return rc;
       vec = vec && vec_ok(hp[i], hs[i], 3, V) && vec_ok(gp[i], gs[i], 3, V);
     }
+  }
+  // values and their gradient in 16-byte vectors too, or both in
+  // time-contiguous rows
+  int rm = ROWS_NONE;
+  if (vec && !(vec_ok(u.p, u.s, 3, V) && vec_ok(du.p, du.s, 3, V))) {
+    const int ru = rows_mode(dtype, u.p, u.s, T, D, r);
+    const int rd = rows_mode(dtype, du.p, du.s, T, D, r);
+    if (look_back_nwin(T, P, Q) == 1 && bwd_gate_mode(r, Da, V) == GATE_LANE &&
+        ru != ROWS_NONE && rd != ROWS_NONE)
+      rm = std::max(ru, rd);
+    vec = rm != ROWS_NONE;
   }
   a.du = to_dev(du);
   a.dlg = to_dev(dlg);
@@ -1075,7 +1118,7 @@ int scan_backward_impl(int dtype, const HostView4& u, const HostView4& lg, const
       f.wst = const_cast<void*>(a.wst);
       f.kw = a.kw;
       const bool fvec = (D % V == 0) && vec_ok(u.p, u.s, 3, V) && vec_ok(init.p, init.s, 3, V);
-      rc = launch_forward(dtype, f, fvec, lg, B, T, NH, NKVH, Da, r, use_sigmoid, st);
+      rc = launch_forward(dtype, f, fvec, ROWS_NONE, lg, B, T, NH, NKVH, Da, r, use_sigmoid, st);
       if (rc) return rc;
     }
     if (gm < 0) {
@@ -1091,7 +1134,7 @@ int scan_backward_impl(int dtype, const HostView4& u, const HostView4& lg, const
       cfg.L = tu.bwd_l;
       cfg.NW = tu.bwd_nw;
     }
-    rc = scan_launch_bwd(bf16, a, cfg, (int)grid, vec, gm, true, st);
+    rc = scan_launch_bwd(bf16, a, cfg, (int)grid, vec, gm, true, ROWS_NONE, st);
     if (rc) return rc;
     if (a.kw > 0) {
       rc = scan_launch_lb_fold(bf16, a, st);
@@ -1104,7 +1147,10 @@ int scan_backward_impl(int dtype, const HostView4& u, const HostView4& lg, const
   if (gm >= 0 && vec && chain_ws != nullptr) {
     // chained: one tile per chunk, the carries handed between workgroups
     const BwdChainPlan pl = bwd_chain_plan(dtype, B, T, H, Da, r);
-    if (pl.cfg.CL > 0 && pl.gm == gm) {
+    // the row modes are built for the default chained shapes
+    const bool rows_ok =
+        rm == ROWS_NONE || (pl.cfg.L == 4 && pl.cfg.NW == 4 && pl.cfg.CL <= 32);
+    if (pl.cfg.CL > 0 && pl.gm == gm && rows_ok) {
       LTV_REQUIRE(chain_ws_bytes >= pl.bytes, LTV_ERR_WORKSPACE,
                   "chained scan workspace too small: %zu bytes, need %zu", chain_ws_bytes,
                   pl.bytes);
@@ -1119,7 +1165,7 @@ int scan_backward_impl(int dtype, const HostView4& u, const HostView4& lg, const
       a.ch_words = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(chain_ws) +
                                                          kChainHeader);
       a.ch_ctl = chain_ctl(st);
-      rc = scan_launch_bwd_chain(dtype == LTV_DTYPE_BF16, a, pl.cfg, (int)grid, gm, st);
+      rc = scan_launch_bwd_chain(dtype == LTV_DTYPE_BF16, a, pl.cfg, (int)grid, gm, rm, st);
       if (rc) return rc;
       return scan_launch_dbias_reduce(a.dbias_partial, dbias, B, H, a.nchunk, Da, st, ds, pz);
     }
@@ -1128,7 +1174,9 @@ int scan_backward_impl(int dtype, const HostView4& u, const HostView4& lg, const
     // whole head per workgroup
     ScanCfg cfg = bwd_tile_cfg(next_pow2((D + V - 1) / V), vec, (int64_t)B * H);
     const ScanTuning& tu = tuning();
-    if (vec && tu.bwd_l > 0) {
+    if (rm != ROWS_NONE) {
+      cfg.L = cfg.NW = 4;
+    } else if (vec && tu.bwd_l > 0) {
       cfg.L = tu.bwd_l;
       cfg.NW = tu.bwd_nw;
     }
@@ -1152,7 +1200,7 @@ int scan_backward_impl(int dtype, const HostView4& u, const HostView4& lg, const
       rc = scan_launch_bwd_chunk_maps(dtype == LTV_DTYPE_BF16, a, vec, st);
       if (rc) return rc;
     }
-    rc = scan_launch_bwd(dtype == LTV_DTYPE_BF16, a, cfg, (int)grid, vec, gm, false, st);
+    rc = scan_launch_bwd(dtype == LTV_DTYPE_BF16, a, cfg, (int)grid, vec, gm, false, rm, st);
     if (rc) return rc;
   } else {
     LTV_REQUIRE((int64_t)B * H < (1ll << 31), LTV_ERR_UNSUPPORTED, "grid too large");

@@ -2,11 +2,12 @@
 #include "ltv_scan_launch.hpp"
 
 namespace ltv {
-int scan_bwd_launch_f32(const BwdArgs& a, ScanCfg c, int grid, bool vec, int gm, bool lb,
+int scan_bwd_launch_f32(const BwdArgs& a, ScanCfg c, int grid, bool vec, int gm, bool lb, int rm,
                         hipStream_t st) {
-  return scan_bwd_launch_t<float>(a, c, grid, vec, gm, lb, st);
+  return scan_bwd_launch_t<float>(a, c, grid, vec, gm, lb, rm, st);
 }
-int scan_bwd_chain_launch_f32(const BwdArgs& a, ScanCfg c, int grid, int gm, hipStream_t st) {
-  return scan_bwd_chain_launch_t<float>(a, c, grid, gm, st);
+int scan_bwd_chain_launch_f32(const BwdArgs& a, ScanCfg c, int grid, int gm, int rm,
+                              hipStream_t st) {
+  return scan_bwd_chain_launch_t<float>(a, c, grid, gm, rm, st);
 }
 }  // namespace ltv

@@ -648,9 +648,228 @@ struct LogitRaw {
 };
 
 // ---------------------------------------------------------------------------
+// A lane's packed values of one tile: V channels x L steps
+// ---------------------------------------------------------------------------
+// How the value slots lie in memory:
+//   ROWS_NONE  channel-contiguous (or element-wise) steps: one vector per step;
+//   ROWS_EVEN  time-contiguous rows, one per channel, as in the transposed view
+//              of a (B, F, T) projection: every row starts on a dword and T is a
+//              multiple of 4, so a row's 4 steps are one 8-byte (bf16) or
+//              16-byte (fp32) access;
+//   ROWS_ANY   time-contiguous rows of any T >= 4 and any alignment.
+// One element per access, the only other way to read such a view, is bound by
+// its own instructions and by the L2's requests for 2- and 4-byte pieces of
+// lines: at B = 16, T = 1024, 18 heads of 128 in bf16 the forward ran at 1.5 and
+// the backward at 0.6 TB/s.  In quads a lane keeps its L x V elements in as many
+// registers, a wavefront's access touches 64 / TG rows of TG x 4 steps, and the
+// workgroup's four wavefronts cover whole 128-byte lines: 4.1 and 2.6 TB/s
+// (103 -> 37 us, 365 -> 88 us).
+enum RowMode { ROWS_NONE = 0, ROWS_EVEN = 1, ROWS_ANY = 2 };
+
+// ROWS_NONE: one packed vector of V channels per step, loaded by the kernels.
+template <typename TIO, bool VEC, int L, int RM>
+struct UTile {
+  uint4 q[L];
+  __device__ __forceinline__ void settle(const char*, int, int, uint32_t, int) {}
+  __device__ __forceinline__ float get(int s, int v) const { return Pack<TIO>::get(q[s], v); }
+  __device__ __forceinline__ void reload() { reload_barrier(q); }
+};
+
+// Time-contiguous rows: row v (channel c0 + v) as NQ quads of 4 steps.
+template <typename TIO, int L, int RM>
+struct RowTile {
+  static_assert(L % 4 == 0, "whole quads of steps");
+  static constexpr int V = Pack<TIO>::V;
+  static constexpr int E = sizeof(TIO);
+  static constexpr int NQ = L / 4;
+  static constexpr int QW = E;  // dwords per quad: 2 (bf16) or 4 (fp32)
+  // ROWS_ANY bf16 rows may start inside a dword: a third dword per quad holds
+  // the piece that spills over until settle() aligns the row
+  static constexpr int RW = RM == ROWS_ANY && E == 2 ? 3 : QW;
+  uint32_t w[V][NQ][RW];
+
+  // Rows of the (b, h) slice at bh, tile at Tt, lane's first step Tt + tl0 at
+  // byte offset off of the tile, scb bytes between rows.  Steps at or past T
+  // read 0.
+  // ROWS_ANY: the last quad of a row is read from T - 4 on, never past the
+  // row's end, and settle() shifts it into place.
+  template <int AUX>
+  __device__ __forceinline__ void load(const char* bh, int Tt, int tl0, uint32_t off,
+                                       uint32_t scb, int T, bool ok) {
+    if constexpr (RM == ROWS_EVEN) {
+      const Rsrc r = make_rsrc(bh + (int64_t)Tt * E);
+#pragma unroll
+      for (int v = 0; v < V; ++v)
+#pragma unroll
+        for (int k = 0; k < NQ; ++k)
+          ldq<AUX>(r, ok && Tt + tl0 + 4 * k < T ? off + v * scb + 4 * k * E : kOob, w[v][k]);
+    } else {
+      // the buffer starts 4 steps before the tile (T >= 4, so that no offset
+      // is negative), on a dword
+      const char* base = bh + ((int64_t)Tt - 4) * E;
+      const uint32_t pb = E == 2 ? (uint32_t)(reinterpret_cast<uintptr_t>(base) & 2u) : 0u;
+      const Rsrc r = make_rsrc(base - pb);
+      const uint32_t chan = off - (uint32_t)(tl0 * E);
+#pragma unroll
+      for (int v = 0; v < V; ++v)
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) {
+          const int t = Tt + tl0 + 4 * k;
+          const bool in = ok && t < T;
+          const uint32_t o = (uint32_t)((min(t, T - 4) - Tt + 4) * E) + chan + v * scb + pb;
+          if constexpr (E == 2) {
+            const uint32_t o4 = o & ~3u;
+            ldq<AUX>(r, in ? o4 : kOob, w[v][k]);
+            w[v][k][2] = __builtin_amdgcn_raw_buffer_load_b32(r, in && (o & 2u) ? o4 + 8u : kOob,
+                                                              0, AUX);
+          } else {
+            ldq<AUX>(r, in ? o : kOob, w[v][k]);
+          }
+        }
+    }
+  }
+
+  // ROWS_ANY: aligns the loaded rows (called where the tile is used, so that
+  // nothing waits for the loads before).
+  __device__ __forceinline__ void settle(const char* bh, int Tt, int tl0, uint32_t scb, int T) {
+    if constexpr (RM == ROWS_ANY) {
+      const char* base = bh + ((int64_t)Tt - 4) * E;
+      const uint32_t pb = E == 2 ? (uint32_t)(reinterpret_cast<uintptr_t>(base) & 2u) : 0u;
+#pragma unroll
+      for (int k = 0; k < NQ; ++k) {
+        const int t = Tt + tl0 + 4 * k;
+        const int tl = min(t, T - 4);
+        const int sh = t - tl;  // steps the quad was read early; > 3: past T, all zeros
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          if constexpr (E == 2) {
+            const uint32_t mis =
+                (((uint32_t)((tl - Tt + 4) * E) + v * scb + pb) & 2u) << 3;
+            const uint32_t lo = __builtin_amdgcn_alignbit(w[v][k][1], w[v][k][0], mis);
+            const uint32_t hi = __builtin_amdgcn_alignbit(w[v][k][2], w[v][k][1], mis);
+            const uint64_t x = (((uint64_t)hi << 32) | lo) >> (16 * (sh & 3));
+            w[v][k][0] = (uint32_t)x;
+            w[v][k][1] = (uint32_t)(x >> 32);
+          } else {
+            uint32_t(&q)[RW] = w[v][k];
+            if (sh & 1) {
+              q[0] = q[1];
+              q[1] = q[2];
+              q[2] = q[3];
+              q[3] = 0u;
+            }
+            if (sh & 2) {
+              q[0] = q[2];
+              q[1] = q[3];
+              q[2] = 0u;
+              q[3] = 0u;
+            }
+          }
+        }
+      }
+    }
+  }
+
+  __device__ __forceinline__ float get(int s, int v) const {
+    if constexpr (E == 2) {
+      const uint32_t x = w[v][s >> 2][(s & 3) >> 1];
+      return __uint_as_float((s & 1) ? (x & 0xffff0000u) : (x << 16));
+    } else {
+      return __uint_as_float(w[v][s >> 2][s & 3]);
+    }
+  }
+  __device__ __forceinline__ void reload() {
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+#pragma unroll
+      for (int k = 0; k < NQ; ++k)
+#pragma unroll
+        for (int i = 0; i < QW; ++i) asm volatile("" : "+v"(w[v][k][i]));
+  }
+
+ private:
+  template <int AUX>
+  __device__ static __forceinline__ void ldq(Rsrc r, uint32_t off, uint32_t (&o)[RW]) {
+    if constexpr (E == 2) {
+      const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, AUX));
+      o[0] = x.x;
+      o[1] = x.y;
+    } else {
+      const uint4 x = bld128<AUX>(r, off);
+      o[0] = x.x;
+      o[1] = x.y;
+      o[2] = x.z;
+      o[3] = x.w;
+    }
+  }
+};
+template <typename TIO, bool VEC, int L>
+struct UTile<TIO, VEC, L, ROWS_EVEN> : RowTile<TIO, L, ROWS_EVEN> {};
+template <typename TIO, bool VEC, int L>
+struct UTile<TIO, VEC, L, ROWS_ANY> : RowTile<TIO, L, ROWS_ANY> {};
+
+// One lane's V rows of L steps, x[s][v], to time-contiguous rows: bh the (b, h)
+// slice, off the lane's byte offset in the tile at Tt (first step Tt + tl0, TW
+// steps per tile), scb bytes between rows.  Steps at or past T are not written.
+// ROWS_ANY: a row that starts inside a dword stores its outer steps as single
+// elements; the tile with the end of T stores every step by itself.  The
+// branches are uniform over the wavefront (c0 is a multiple of V, tl0 of 4).
+template <typename TIO, int L, int RM, int TW>
+__device__ __forceinline__ void st_rows(const char* bh, int Tt, int tl0, uint32_t off,
+                                        uint32_t scb, int T, bool ok,
+                                        const float (&x)[L][Pack<TIO>::V]) {
+  constexpr int V = Pack<TIO>::V;
+  constexpr int E = sizeof(TIO);
+  const char* base = bh + (int64_t)Tt * E;
+  const Rsrc r = make_rsrc(base);
+  auto whole = [&](int v, int k, bool in) {
+    const uint32_t o = in ? off + v * scb + 4 * k * E : kOob;
+    if constexpr (E == 2) {
+      typedef int i32x2_t __attribute__((ext_vector_type(2)));
+      const i32x2_t d = {(int)cvt_pk_bf16(x[4 * k][v], x[4 * k + 1][v]),
+                         (int)cvt_pk_bf16(x[4 * k + 2][v], x[4 * k + 3][v])};
+      __builtin_amdgcn_raw_buffer_store_b64(d, r, o, 0, kStNormal);
+    } else {
+      bst128(r, o, make_uint4(__float_as_uint(x[4 * k][v]), __float_as_uint(x[4 * k + 1][v]),
+                              __float_as_uint(x[4 * k + 2][v]), __float_as_uint(x[4 * k + 3][v])));
+    }
+  };
+  if constexpr (RM == ROWS_EVEN) {
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+#pragma unroll
+      for (int k = 0; k < L / 4; ++k) whole(v, k, ok && Tt + tl0 + 4 * k < T);
+  } else if (Tt + TW <= T) {
+    const uint32_t b0 = (uint32_t)reinterpret_cast<uintptr_t>(base);
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+#pragma unroll
+      for (int k = 0; k < L / 4; ++k) {
+        if (E == 4 || ((b0 + v * scb) & 2u) == 0u) {
+          whole(v, k, ok);
+        } else {
+          const uint32_t o = off + v * scb + 4 * k * E;
+          bst1<TIO>(r, ok ? o : kOob, x[4 * k][v]);
+          bst_b32(r, ok ? o + 2u : kOob,
+                  __uint_as_float(cvt_pk_bf16(x[4 * k + 1][v], x[4 * k + 2][v])));
+          bst1<TIO>(r, ok ? o + 6u : kOob, x[4 * k + 3][v]);
+        }
+      }
+  } else {
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+#pragma unroll
+      for (int s = 0; s < L; ++s)
+        bst1<TIO>(r, ok && Tt + tl0 + s < T ? off + v * scb + s * E : kOob, x[s][v]);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Forward
 // ---------------------------------------------------------------------------
-template <typename TIO, int CL, int L, int NW, bool VEC, int GM>
+// RM: how the values lie (RowMode); the row modes run the full recurrence with
+// one gate per lane and 16-byte vectors everywhere else (VEC).
+template <typename TIO, int CL, int L, int NW, bool VEC, int GM, int RM = ROWS_NONE>
 __global__ void __launch_bounds__(NW * 64)
 scan_fwd_kernel(const FwdArgs args) {
   constexpr int V = Pack<TIO>::V;
@@ -737,16 +956,21 @@ scan_fwd_kernel(const FwdArgs args) {
   // use two buffers (with one, the compiler copies the new loads into the
   // body's registers at the end of each tile, waiting there for every
   // outstanding memory operation, the tile's stores included)
-  uint4 nu[2][L];
+  UTile<TIO, VEC, L, RM> nu[2];
   LogitRaw<TIO, GM, L> nl[2];
   auto load_tile = [&](int it, auto bufc) {
     constexpr int buf = decltype(bufc)::value;
     const int Tt = t_lo + it * TW;
     const int t0 = Tt + tl0;
-    const Rsrc ur = make_rsrc(ubh + (int64_t)Tt * args.u.s[2] * E);
+    if constexpr (RM != ROWS_NONE) {
+      nu[buf].template load<kLdNormal>(ubh, Tt, tl0, uoff, uscb, t_hi, active);
+    } else {
+      const Rsrc ur = make_rsrc(ubh + (int64_t)Tt * args.u.s[2] * E);
 #pragma unroll
-    for (int s = 0; s < L; ++s)
-      nu[buf][s] = bld_vec<TIO, VEC>(ur, uoff + s * ustb, uscb, nvalid, active && (t0 + s) < t_hi);
+      for (int s = 0; s < L; ++s)
+        nu[buf].q[s] =
+            bld_vec<TIO, VEC>(ur, uoff + s * ustb, uscb, nvalid, active && (t0 + s) < t_hi);
+    }
     nl[buf].load(make_rsrc(lbh + (int64_t)Tt * args.lg.s[2] * E), loff, lstb, gi, t0, t_hi,
                  active, nvalid);
   };
@@ -755,9 +979,8 @@ scan_fwd_kernel(const FwdArgs args) {
     constexpr int buf = decltype(bufc)::value;
     const int Tt = t_lo + it * TW;
     const int t0 = Tt + tl0;
-    uint4 uq[L];
-#pragma unroll
-    for (int s = 0; s < L; ++s) uq[s] = nu[buf][s];
+    UTile<TIO, VEC, L, RM> uq = nu[buf];
+    uq.settle(ubh, Tt, tl0, uscb, t_hi);
     float al[L][NA];
     nl[buf].gates(gi, t0, t_hi, active, use_sig, al);
     // past the end: every lane masked, no memory access
@@ -774,7 +997,7 @@ scan_fwd_kernel(const FwdArgs args) {
 #pragma unroll
       for (int v = 0; v < V; ++v) {
         const float a = al[s][GL ? 0 : v];
-        X[v] = fmaf(a, Pack<TIO>::get(uq[s], v) - X[v], X[v]);
+        X[v] = fmaf(a, uq.get(s, v) - X[v], X[v]);
       }
 #pragma unroll
       for (int i = 0; i < NA; ++i) A[i] = fmaf(-A[i], al[s][i], A[i]);
@@ -827,7 +1050,7 @@ scan_fwd_kernel(const FwdArgs args) {
     }
 
     // re-run the lane's steps from its exact carry-in and store
-    reload_barrier(uq);
+    uq.reload();
     const Rsrc orr = make_rsrc(obh + (int64_t)Tt * ost * E);
     float hv[V];
 #pragma unroll
@@ -837,7 +1060,7 @@ scan_fwd_kernel(const FwdArgs args) {
 #pragma unroll
       for (int v = 0; v < V; ++v) {
         const float a = al[s][GL ? 0 : v];
-        hv[v] = fmaf(a, Pack<TIO>::get(uq[s], v) - hv[v], hv[v]);
+        hv[v] = fmaf(a, uq.get(s, v) - hv[v], hv[v]);
       }
       bst_vec<TIO, VEC, GM == GATE_CHANVEC ? kStStream : kStNormal>(
           orr, ooff + s * ostb, oscb, nvalid, active && (t0 + s) >= t_st && (t0 + s) < t_hi, hv);
@@ -959,7 +1182,7 @@ __device__ __forceinline__ void chain_clear_abandoned(unsigned long long* pw,
   if (prev != 0ull) __hip_atomic_store(pw, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <typename TIO, int CL, int L, int NW, bool VEC, int GM>
+template <typename TIO, int CL, int L, int NW, bool VEC, int GM, int RM = ROWS_NONE>
 __global__ void __launch_bounds__(NW * 64)
 scan_fwd_chain_kernel(const FwdArgs args, const ChainArgs ch) {
   constexpr int V = Pack<TIO>::V;
@@ -1036,13 +1259,17 @@ scan_fwd_chain_kernel(const FwdArgs args, const ChainArgs ch) {
   const uint32_t ooff = (uint32_t)tl0 * ostb + (uint32_t)c0 * oscb;
 
   // the whole chunk is loaded at once: L vectors and logits per lane in flight
-  uint4 uq[L];
+  UTile<TIO, VEC, L, RM> uq;
   LogitRaw<TIO, GM, L> lr;
   {
     const Rsrc ur = make_rsrc(ubh + (int64_t)Tt * args.u.s[2] * E);
+    if constexpr (RM != ROWS_NONE) {
+      uq.template load<kLdNormal>(ubh, Tt, tl0, uoff, uscb, T, active);
+    } else {
 #pragma unroll
-    for (int s = 0; s < L; ++s)
-      uq[s] = bld_vec<TIO, VEC>(ur, uoff + s * ustb, uscb, nvalid, active && (t0 + s) < T);
+      for (int s = 0; s < L; ++s)
+        uq.q[s] = bld_vec<TIO, VEC>(ur, uoff + s * ustb, uscb, nvalid, active && (t0 + s) < T);
+    }
     lr.load(make_rsrc(lbh + (int64_t)Tt * args.lg.s[2] * E), loff, lstb, gi, t0, T, active,
             nvalid);
   }
@@ -1061,6 +1288,7 @@ scan_fwd_chain_kernel(const FwdArgs args, const ChainArgs ch) {
 
   float al[L][NA];
   lr.gates(gi, t0, T, active, use_sig, al);
+  uq.settle(ubh, Tt, tl0, uscb, T);
 
   // level 1: lane-local fold (padded steps have alpha = 0: the identity)
   float A[NA], X[V];
@@ -1073,7 +1301,7 @@ scan_fwd_chain_kernel(const FwdArgs args, const ChainArgs ch) {
 #pragma unroll
     for (int v = 0; v < V; ++v) {
       const float a = al[s][GL ? 0 : v];
-      X[v] = fmaf(a, Pack<TIO>::get(uq[s], v) - X[v], X[v]);
+      X[v] = fmaf(a, uq.get(s, v) - X[v], X[v]);
     }
 #pragma unroll
     for (int i = 0; i < NA; ++i) A[i] = fmaf(-A[i], al[s][i], A[i]);
@@ -1153,7 +1381,7 @@ scan_fwd_chain_kernel(const FwdArgs args, const ChainArgs ch) {
   }
 
   // re-run the lane's steps from its exact carry-in and store
-  reload_barrier(uq);
+  uq.reload();
   const Rsrc orr = make_rsrc(obh + (int64_t)Tt * ov.s[2] * E);
   float hv[V];
 #pragma unroll
@@ -1163,7 +1391,7 @@ scan_fwd_chain_kernel(const FwdArgs args, const ChainArgs ch) {
 #pragma unroll
     for (int v = 0; v < V; ++v) {
       const float a = al[s][GL ? 0 : v];
-      hv[v] = fmaf(a, Pack<TIO>::get(uq[s], v) - hv[v], hv[v]);
+      hv[v] = fmaf(a, uq.get(s, v) - hv[v], hv[v]);
     }
     bst_vec<TIO, VEC, GM == GATE_CHANVEC ? kStStream : kStNormal>(
         orr, ooff + s * ostb, oscb, nvalid, active && (t0 + s) < T, hv);
@@ -1191,7 +1419,9 @@ constexpr int kMaxLaneGroups = 16;
 // with the same launch shape.  Deadlock-free for the chained forward's
 // reason: a workgroup waits only for a smaller ticket, drawn by a workgroup
 // that is already running.
-template <typename TIO, int CL, int L, int NW, bool VEC, int GM, bool LB, bool CHAIN = false>
+// RM: how the values and their gradients lie (RowMode; both alike).
+template <typename TIO, int CL, int L, int NW, bool VEC, int GM, bool LB, bool CHAIN = false,
+          int RM = ROWS_NONE>
 __global__ void __launch_bounds__(NW * 64)
 scan_bwd_kernel(const BwdArgs args) {
   constexpr int V = Pack<TIO>::V;
@@ -1202,6 +1432,7 @@ scan_bwd_kernel(const BwdArgs args) {
   constexpr int NCH = CL * V;  // chained mode: one carry word per channel slot
   constexpr bool GL = GM == GATE_LANE;
   static_assert(!(CHAIN && LB), "the chained backward runs the full recurrence");
+  static_assert(RM == ROWS_NONE || (VEC && GL && !LB), "row modes: one gate per lane, no windows");
   static_assert(!CHAIN || NCH <= NT, "the chain step takes one thread per channel slot");
   const ScanShape& S = args.sh;
 
@@ -1358,7 +1589,8 @@ scan_bwd_kernel(const BwdArgs args) {
   // the state entering the lane comes from one of three masked loads, kept
   // apart until the tile uses it (merging them at once would wait for the
   // loads just issued)
-  uint4 nu[NB][L], ng[NB][L], nh0[NB], nw0[LB ? NB : 1];
+  UTile<TIO, VEC, L, RM> nu[NB];
+  uint4 ng[NB][L], nh0[NB], nw0[LB ? NB : 1];
   // The inits of this lane's channels are read once, here, raw (16-byte
   // vectors; fp32 inits with bf16 I/O are two), and converted by selects in
   // the tile whose lane starts at t_base: a branch on the dtype inside the
@@ -1394,11 +1626,14 @@ scan_bwd_kernel(const BwdArgs args) {
     const bool tile_ok = active && it >= it_lo;
     const Rsrc ur = make_rsrc(ubh + (int64_t)Tt * args.u.s[2] * E);
     const Rsrc gr = make_rsrc(gbh + (int64_t)Tt * gs[2] * E);
+    if constexpr (RM != ROWS_NONE)
+      nu[buf].template load<kLdStream>(ubh, Tt, tl0, uoff, uscb, t_hi, tile_ok);
 #pragma unroll
     for (int s = 0; s < L; ++s) {
       const int t = t0 + s;
       const bool ok = tile_ok && t < t_hi;
-      nu[buf][s] = bld_vec<TIO, VEC, kLdStream>(ur, uoff + s * ustb, uscb, nvalid, ok);
+      if constexpr (RM == ROWS_NONE)
+        nu[buf].q[s] = bld_vec<TIO, VEC, kLdStream>(ur, uoff + s * ustb, uscb, nvalid, ok);
       ng[buf][s] = bld_vec<TIO, VEC, kLdStream>(gr, goff + s * gstb, gscb, nvalid,
                                                 ok && (!LB || t >= t_st));
     }
@@ -1433,12 +1668,11 @@ scan_bwd_kernel(const BwdArgs args) {
     const int T0 = t_base + it * TW;
     const int t0 = T0 + tl0;
 
-    uint4 uq[L], gq[L], hq[L];
+    UTile<TIO, VEC, L, RM> uq = nu[buf];
+    uq.settle(ubh, T0, tl0, uscb, t_hi);
+    uint4 gq[L], hq[L];
 #pragma unroll
-    for (int s = 0; s < L; ++s) {
-      uq[s] = nu[buf][s];
-      gq[s] = ng[buf][s];
-    }
+    for (int s = 0; s < L; ++s) gq[s] = ng[buf][s];
     {
       uint4 q = nh0[buf];
       // the lane that starts at t_base enters from the inits (its h load was
@@ -1464,7 +1698,7 @@ scan_bwd_kernel(const BwdArgs args) {
 #pragma unroll
       for (int v = 0; v < V; ++v) {
         const float hp_ = Pack<TIO>::get(hq[s - 1], v);
-        hv[v] = fmaf(al[s - 1][GL ? 0 : v], Pack<TIO>::get(uq[s - 1], v) - hp_, hp_);
+        hv[v] = fmaf(al[s - 1][GL ? 0 : v], uq.get(s - 1, v) - hp_, hp_);
       }
       hq[s] = Pack<TIO>::pack(hv);
     }
@@ -1579,6 +1813,7 @@ scan_bwd_kernel(const BwdArgs args) {
     const Rsrc wdur = make_rsrc(LB ? wdubh + (int64_t)(T0 - t_base) * S.D * 4 : dubh);
     const Rsrc wdlr = make_rsrc(LB ? wdlbh + (int64_t)(T0 - t_base) * S.Da * 4 : dlbh);
     float pl[L];  // GATE_LANE: this lane's dalpha partial per step
+    float du_rows[RM != ROWS_NONE ? L : 1][V];  // row modes: stored after the loop
 #pragma unroll
     for (int s = L - 1; s >= 0; --s) {
       const int t = t0 + s;
@@ -1591,9 +1826,14 @@ scan_bwd_kernel(const BwdArgs args) {
         gv[v] = fmaf(dk[s][ia], gin[v], Pack<TIO>::get(gq[s], v));
         gin[v] = gv[v];
         duv[v] = al[s][ia] * gv[v];
-        dav[v] = (Pack<TIO>::get(uq[s], v) - Pack<TIO>::get(hq[s], v)) * gv[v];
+        dav[v] = (uq.get(s, v) - Pack<TIO>::get(hq[s], v)) * gv[v];
       }
-      bst_vec<TIO, VEC>(dur, duoff + s * dustb, duscb, nvalid, ok && !wu, duv);
+      if constexpr (RM != ROWS_NONE) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) du_rows[s][v] = duv[v];
+      } else {
+        bst_vec<TIO, VEC>(dur, duoff + s * dustb, duscb, nvalid, ok && !wu, duv);
+      }
       if (LB) bst_f32<VEC, V>(wdur, wduoff + s * wdustb, nvalid, ok && wu, duv);
       if (GL) {
         float p = 0.0f;
@@ -1642,6 +1882,8 @@ scan_bwd_kernel(const BwdArgs args) {
         }
       }
     }
+    if constexpr (RM != ROWS_NONE)
+      st_rows<TIO, L, RM, TW>(dubh, T0, tl0, duoff, duscb, t_hi, active, du_rows);
     // kept from the last tile processed (it_lo), whose lane tl0 == 0 holds t_base
 #pragma unroll
     for (int v = 0; v < V; ++v) dinit_v[v] = (1.0f - al[0][GL ? 0 : v]) * gin[v];
@@ -2139,19 +2381,21 @@ struct ScanCfg {
 };
 
 // Forward: grid = B * H * nslab workgroups of NW * 64 threads.
-int scan_launch_fwd(bool bf16, const FwdArgs& a, ScanCfg cfg, int grid, bool vec, int gm,
+// rm: RowMode of the values (ROWS_EVEN / ROWS_ANY with vec: every other view
+// in 16-byte vectors).
+int scan_launch_fwd(bool bf16, const FwdArgs& a, ScanCfg cfg, int grid, bool vec, int gm, int rm,
                     hipStream_t st);
 // Forward with chained chunk states: grid = nseq * nchunk workgroups (vector
 // accesses only; gate modes GATE_LANE and GATE_CHANVEC).
 int scan_launch_fwd_chain(bool bf16, const FwdArgs& a, const ChainArgs& ch, ScanCfg cfg, int gm,
-                          hipStream_t st);
+                          int rm, hipStream_t st);
 // Backward main kernel: grid = B * H * nchunk; CL channel lanes cover the whole
 // head; lb selects the look-back window kernels.
 int scan_launch_bwd(bool bf16, const BwdArgs& a, ScanCfg cfg, int grid, bool vec, int gm,
-                    bool lb, hipStream_t st);
+                    bool lb, int rm, hipStream_t st);
 // Chained backward: grid = B * H * nchunk workgroups, one tile per chunk
 // (vector accesses only; gate modes GATE_LANE and GATE_CHANVEC).
-int scan_launch_bwd_chain(bool bf16, const BwdArgs& a, ScanCfg cfg, int grid, int gm,
+int scan_launch_bwd_chain(bool bf16, const BwdArgs& a, ScanCfg cfg, int grid, int gm, int rm,
                           hipStream_t st);
 // Look-back backward: warm-up contributions into du / dlg, then grad_inits.
 int scan_launch_lb_fold(bool bf16, const BwdArgs& a, hipStream_t st);

@@ -18,9 +18,29 @@ constexpr bool is_base_cfg() {
   return L == 4 && NW == 4;
 }
 
+// The shapes the row modes are built for: heads of 32, 64 and 128 channels with
+// 16-byte vectors (forward slabs of up to 8 channel lanes, whole heads in the
+// backward), 4 steps per lane and wavefront counts that make a tile's rows
+// whole 128-byte lines.
+template <int CL, int L, int NW>
+constexpr bool is_rows_cfg() {
+  return L == 4 && NW == 4 && CL >= 4 && CL <= 32;
+}
+
 template <typename TIO, int CL, int L, int NW>
-bool fwd_dispatch(const FwdArgs& a, int grid, bool vec, int gm, hipStream_t st) {
+bool fwd_dispatch(const FwdArgs& a, int grid, bool vec, int gm, int rm, hipStream_t st) {
   const dim3 blk(NW * 64);
+  if (rm != ROWS_NONE) {
+    if constexpr (is_rows_cfg<CL, L, NW>() && CL <= 8) {
+      if (!vec || gm != GATE_LANE) return false;
+      if (rm == ROWS_EVEN)
+        hipLaunchKernelGGL((scan_fwd_kernel<TIO, CL, L, NW, true, GATE_LANE, ROWS_EVEN>), dim3(grid), blk, 0, st, a);
+      else
+        hipLaunchKernelGGL((scan_fwd_kernel<TIO, CL, L, NW, true, GATE_LANE, ROWS_ANY>), dim3(grid), blk, 0, st, a);
+      return true;
+    }
+    return false;
+  }
   if (vec) {
     switch (gm) {
       case GATE_LANE:
@@ -52,8 +72,20 @@ bool fwd_dispatch(const FwdArgs& a, int grid, bool vec, int gm, hipStream_t st) 
 }
 
 template <typename TIO, int CL, int L, int NW>
-bool fwd_chain_dispatch(const FwdArgs& a, const ChainArgs& ch, int grid, int gm, hipStream_t st) {
+bool fwd_chain_dispatch(const FwdArgs& a, const ChainArgs& ch, int grid, int gm, int rm,
+                        hipStream_t st) {
   const dim3 blk(NW * 64);
+  if (rm != ROWS_NONE) {
+    if constexpr (CL == 8 && L == 8 && NW == 8) {  // the default shape
+      if (gm != GATE_LANE) return false;
+      if (rm == ROWS_EVEN)
+        hipLaunchKernelGGL((scan_fwd_chain_kernel<TIO, CL, L, NW, true, GATE_LANE, ROWS_EVEN>), dim3(grid), blk, 0, st, a, ch);
+      else
+        hipLaunchKernelGGL((scan_fwd_chain_kernel<TIO, CL, L, NW, true, GATE_LANE, ROWS_ANY>), dim3(grid), blk, 0, st, a, ch);
+      return true;
+    }
+    return false;
+  }
   switch (gm) {
     case GATE_LANE:
       hipLaunchKernelGGL((scan_fwd_chain_kernel<TIO, CL, L, NW, true, GATE_LANE>), dim3(grid), blk, 0, st, a, ch);
@@ -107,15 +139,38 @@ bool bwd_dispatch_lb(const BwdArgs& a, int grid, bool vec, int gm, hipStream_t s
 }
 
 template <typename TIO, int CL, int L, int NW>
-bool bwd_dispatch(const BwdArgs& a, int grid, bool vec, int gm, bool lb, hipStream_t st) {
+bool bwd_dispatch(const BwdArgs& a, int grid, bool vec, int gm, bool lb, int rm, hipStream_t st) {
+  if (rm != ROWS_NONE) {
+    if constexpr (is_rows_cfg<CL, L, NW>()) {
+      const dim3 blk(NW * 64);
+      if (!vec || gm != GATE_LANE || lb) return false;
+      if (rm == ROWS_EVEN)
+        hipLaunchKernelGGL((scan_bwd_kernel<TIO, CL, L, NW, true, GATE_LANE, false, false, ROWS_EVEN>), dim3(grid), blk, 0, st, a);
+      else
+        hipLaunchKernelGGL((scan_bwd_kernel<TIO, CL, L, NW, true, GATE_LANE, false, false, ROWS_ANY>), dim3(grid), blk, 0, st, a);
+      return true;
+    }
+    return false;
+  }
   if (!lb) return bwd_dispatch_lb<TIO, CL, L, NW, false>(a, grid, vec, gm, st);
   if constexpr (is_lb_cfg<CL, L, NW>()) return bwd_dispatch_lb<TIO, CL, L, NW, true>(a, grid, vec, gm, st);
   return false;
 }
 
 template <typename TIO, int CL, int L, int NW>
-bool bwd_chain_dispatch(const BwdArgs& a, int grid, int gm, hipStream_t st) {
+bool bwd_chain_dispatch(const BwdArgs& a, int grid, int gm, int rm, hipStream_t st) {
   const dim3 blk(NW * 64);
+  if (rm != ROWS_NONE) {
+    if constexpr (is_rows_cfg<CL, L, NW>()) {
+      if (gm != GATE_LANE) return false;
+      if (rm == ROWS_EVEN)
+        hipLaunchKernelGGL((scan_bwd_kernel<TIO, CL, L, NW, true, GATE_LANE, false, true, ROWS_EVEN>), dim3(grid), blk, 0, st, a);
+      else
+        hipLaunchKernelGGL((scan_bwd_kernel<TIO, CL, L, NW, true, GATE_LANE, false, true, ROWS_ANY>), dim3(grid), blk, 0, st, a);
+      return true;
+    }
+    return false;
+  }
   switch (gm) {
     case GATE_LANE:
       hipLaunchKernelGGL((scan_bwd_kernel<TIO, CL, L, NW, true, GATE_LANE, false, true>), dim3(grid), blk, 0, st, a);
@@ -139,11 +194,12 @@ bool bwd_chain_dispatch(const BwdArgs& a, int grid, int gm, hipStream_t st) {
   X(16, 4, 2) X(16, 2, 4)
 
 template <typename TIO>
-int scan_fwd_launch_t(const FwdArgs& a, ScanCfg c, int grid, bool vec, int gm, hipStream_t st) {
+int scan_fwd_launch_t(const FwdArgs& a, ScanCfg c, int grid, bool vec, int gm, int rm,
+                      hipStream_t st) {
   bool ok = false;
 #define LTV_X(CL_, L_, NW_)                                                   \
   if (!ok && c.CL == CL_ && c.L == L_ && c.NW == NW_)                         \
-    ok = detail::fwd_dispatch<TIO, CL_, L_, NW_>(a, grid, vec, gm, st);
+    ok = detail::fwd_dispatch<TIO, CL_, L_, NW_>(a, grid, vec, gm, rm, st);
   LTV_SCAN_FWD_CONFIGS(LTV_X)
 #undef LTV_X
   if (!ok) {
@@ -161,7 +217,7 @@ int scan_fwd_launch_t(const FwdArgs& a, ScanCfg c, int grid, bool vec, int gm, h
   X(8, 16, 4) X(8, 8, 4) X(8, 8, 8) X(8, 4, 4) X(8, 4, 8) X(8, 2, 4)
 
 template <typename TIO>
-int scan_fwd_chain_launch_t(const FwdArgs& a, const ChainArgs& ch, ScanCfg c, int gm,
+int scan_fwd_chain_launch_t(const FwdArgs& a, const ChainArgs& ch, ScanCfg c, int gm, int rm,
                             hipStream_t st) {
   const int64_t grid = (int64_t)ch.nseq * ch.nchunk;
   if (grid <= 0 || grid >= (1ll << 31)) {
@@ -171,7 +227,7 @@ int scan_fwd_chain_launch_t(const FwdArgs& a, const ChainArgs& ch, ScanCfg c, in
   bool ok = false;
 #define LTV_X(CL_, L_, NW_)                                                   \
   if (!ok && c.CL == CL_ && c.L == L_ && c.NW == NW_)                         \
-    ok = detail::fwd_chain_dispatch<TIO, CL_, L_, NW_>(a, ch, (int)grid, gm, st);
+    ok = detail::fwd_chain_dispatch<TIO, CL_, L_, NW_>(a, ch, (int)grid, gm, rm, st);
   LTV_SCAN_FWD_CHAIN_CONFIGS(LTV_X)
 #undef LTV_X
   if (!ok) {
@@ -184,12 +240,12 @@ int scan_fwd_chain_launch_t(const FwdArgs& a, const ChainArgs& ch, ScanCfg c, in
 }
 
 template <typename TIO>
-int scan_bwd_launch_t(const BwdArgs& a, ScanCfg c, int grid, bool vec, int gm, bool lb,
+int scan_bwd_launch_t(const BwdArgs& a, ScanCfg c, int grid, bool vec, int gm, bool lb, int rm,
                       hipStream_t st) {
   bool ok = false;
 #define LTV_X(CL_, L_, NW_)                                                   \
   if (!ok && c.CL == CL_ && c.L == L_ && c.NW == NW_)                         \
-    ok = detail::bwd_dispatch<TIO, CL_, L_, NW_>(a, grid, vec, gm, lb, st);
+    ok = detail::bwd_dispatch<TIO, CL_, L_, NW_>(a, grid, vec, gm, lb, rm, st);
   LTV_SCAN_BWD_CONFIGS(LTV_X)
 #undef LTV_X
   if (!ok) {
@@ -207,12 +263,13 @@ int scan_bwd_launch_t(const BwdArgs& a, ScanCfg c, int grid, bool vec, int gm, b
   X(16, 4, 2) X(16, 4, 4) X(16, 8, 2) X(16, 8, 4) X(16, 2, 4) X(8, 4, 4) X(32, 4, 4) X(32, 4, 2)
 
 template <typename TIO>
-int scan_bwd_chain_launch_t(const BwdArgs& a, ScanCfg c, int grid, int gm, hipStream_t st) {
+int scan_bwd_chain_launch_t(const BwdArgs& a, ScanCfg c, int grid, int gm, int rm,
+                            hipStream_t st) {
   bool ok = false;
 #define LTV_X(CL_, L_, NW_)                                                   \
   if constexpr (CL_ * Pack<TIO>::V <= NW_ * 64)                               \
     if (!ok && c.CL == CL_ && c.L == L_ && c.NW == NW_)                       \
-      ok = detail::bwd_chain_dispatch<TIO, CL_, L_, NW_>(a, grid, gm, st);
+      ok = detail::bwd_chain_dispatch<TIO, CL_, L_, NW_>(a, grid, gm, rm, st);
   LTV_SCAN_BWD_CHAIN_CONFIGS(LTV_X)
 #undef LTV_X
   if (!ok) {
@@ -225,17 +282,21 @@ int scan_bwd_chain_launch_t(const BwdArgs& a, ScanCfg c, int grid, int gm, hipSt
 }
 
 // Per-dtype entry points (defined in the four translation units).
-int scan_fwd_launch_bf16(const FwdArgs& a, ScanCfg c, int grid, bool vec, int gm, hipStream_t st);
-int scan_fwd_launch_f32(const FwdArgs& a, ScanCfg c, int grid, bool vec, int gm, hipStream_t st);
-int scan_fwd_chain_launch_bf16(const FwdArgs& a, const ChainArgs& ch, ScanCfg c, int gm,
-                               hipStream_t st);
-int scan_fwd_chain_launch_f32(const FwdArgs& a, const ChainArgs& ch, ScanCfg c, int gm,
-                              hipStream_t st);
-int scan_bwd_launch_bf16(const BwdArgs& a, ScanCfg c, int grid, bool vec, int gm, bool lb,
+int scan_fwd_launch_bf16(const FwdArgs& a, ScanCfg c, int grid, bool vec, int gm, int rm,
                          hipStream_t st);
-int scan_bwd_launch_f32(const BwdArgs& a, ScanCfg c, int grid, bool vec, int gm, bool lb,
+int scan_fwd_launch_f32(const FwdArgs& a, ScanCfg c, int grid, bool vec, int gm, int rm,
                         hipStream_t st);
-int scan_bwd_chain_launch_bf16(const BwdArgs& a, ScanCfg c, int grid, int gm, hipStream_t st);
-int scan_bwd_chain_launch_f32(const BwdArgs& a, ScanCfg c, int grid, int gm, hipStream_t st);
+int scan_fwd_chain_launch_bf16(const FwdArgs& a, const ChainArgs& ch, ScanCfg c, int gm, int rm,
+                               hipStream_t st);
+int scan_fwd_chain_launch_f32(const FwdArgs& a, const ChainArgs& ch, ScanCfg c, int gm, int rm,
+                              hipStream_t st);
+int scan_bwd_launch_bf16(const BwdArgs& a, ScanCfg c, int grid, bool vec, int gm, bool lb, int rm,
+                         hipStream_t st);
+int scan_bwd_launch_f32(const BwdArgs& a, ScanCfg c, int grid, bool vec, int gm, bool lb, int rm,
+                        hipStream_t st);
+int scan_bwd_chain_launch_bf16(const BwdArgs& a, ScanCfg c, int grid, int gm, int rm,
+                               hipStream_t st);
+int scan_bwd_chain_launch_f32(const BwdArgs& a, ScanCfg c, int grid, int gm, int rm,
+                              hipStream_t st);
 
 }  // namespace ltv
