@@ -1,7 +1,7 @@
 // Fused QKV projection for gfx950: bf16 MFMA GEMMs (fp32 accumulate) for the
 // filter module's fast path, and the reference-layout fused_linear_transpose
 // op (fp32 or bf16 I/O) on the bf16 direct-to-LDS kernels where its layout
-// allows, else on the strided fp32-MFMA GEMM of ltv_gemm_f32.hpp.
+// allows, else (fp32 always) on the strided GEMM of ltv_gemm_split.hpp.
 //
 // Reference: cpp_ewma/src/fused_linear_transpose_forward.cu:23-58 (one
 // strided-batched GEMM, out[b] = W x[b]^T written (B, F, T)) and
@@ -18,7 +18,7 @@
 #include "ltv_device.hpp"
 #include "ltv_abi_internal.hpp"
 #include "ltv_gemm_dma.hpp"
-#include "ltv_gemm_f32.hpp"
+#include "ltv_gemm_split.hpp"
 
 #include <stdio.h>
 #include <stdlib.h>
@@ -201,76 +201,6 @@ using namespace ltv;
 
 namespace {
 
-// Staging form of one operand of the fp32-MFMA GEMM (row stride sr, reduction
-// strides sko / ski, batch stride sbatch): quads need 4-element-aligned
-// starts, and a KQ quad must not straddle two outer reduction indices.
-int f32m_stage(const void* p, int64_t sr, int64_t sko, int64_t ski, int64_t sbatch, int batches,
-               int kin, int K, int esize) {
-  const bool aligned =
-      (reinterpret_cast<uintptr_t>(p) % (uintptr_t)(4 * esize)) == 0 &&
-      (batches <= 1 || sbatch % 4 == 0);
-  const bool outer = kin < K;
-  if (aligned && ski == 1 && sr % 4 == 0 && (!outer || (kin % 4 == 0 && sko % 4 == 0)))
-    return kF32KQ;
-  if (aligned && sr == 1 && ski % 4 == 0 && (!outer || sko % 4 == 0)) return kF32MQ;
-  return kF32SC;
-}
-
-template <typename TI, typename TO, int LA>
-void f32m_launch_b(int lb, const F32mArgs& a, dim3 grid, hipStream_t st) {
-  if (lb == kF32KQ)
-    hipLaunchKernelGGL((gemm_f32m_kernel<TI, TO, LA, kF32KQ>), grid, dim3(kF32Threads), 0, st, a);
-  else if (lb == kF32MQ)
-    hipLaunchKernelGGL((gemm_f32m_kernel<TI, TO, LA, kF32MQ>), grid, dim3(kF32Threads), 0, st, a);
-  else
-    hipLaunchKernelGGL((gemm_f32m_kernel<TI, TO, LA, kF32SC>), grid, dim3(kF32Threads), 0, st, a);
-}
-
-template <typename TI, typename TO>
-void f32m_launch_ab(int la, int lb, const F32mArgs& a, dim3 grid, hipStream_t st) {
-  if (la == kF32KQ)
-    f32m_launch_b<TI, TO, kF32KQ>(lb, a, grid, st);
-  else if (la == kF32MQ)
-    f32m_launch_b<TI, TO, kF32MQ>(lb, a, grid, st);
-  else
-    f32m_launch_b<TI, TO, kF32SC>(lb, a, grid, st);
-}
-
-// C (dtype_out; fp32 for split partials) = A . B^T over `batches` batches and
-// `splits` reduction splits of k_split indices each (splits = 1: k_split is
-// ignored), on the fp32-MFMA GEMM.
-int launch_f32m(int dtype_in, int dtype_out, F32mArgs a, int batches, int splits, int k_split,
-                hipStream_t st) {
-  if (a.M == 0 || a.N == 0 || batches == 0) return LTV_OK;
-  LTV_REQUIRE((dtype_in == LTV_DTYPE_F32 && dtype_out == LTV_DTYPE_F32) ||
-                  (dtype_in == LTV_DTYPE_BF16 &&
-                   (dtype_out == LTV_DTYPE_BF16 || dtype_out == LTV_DTYPE_F32)),
-              LTV_ERR_UNSUPPORTED, "fp32-MFMA GEMM: unsupported dtypes %d -> %d", dtype_in,
-              dtype_out);
-  a.splits = std::max(1, splits);
-  a.k_split = a.splits == 1 ? a.K : k_split;
-  LTV_REQUIRE(a.splits == 1 || (a.k_split > 0 && a.k_split % kF32BK == 0 &&
-                                (int64_t)a.k_split * a.splits >= a.K),
-              LTV_ERR_INVALID_ARG, "bad reduction split (%d x %d for K = %d)", a.splits,
-              a.k_split, a.K);
-  const int64_t gy = (a.M + kF32B - 1) / kF32B, gz = (int64_t)batches * a.splits;
-  LTV_REQUIRE(gy <= 65535 && gz <= 65535, LTV_ERR_UNSUPPORTED,
-              "fp32-MFMA GEMM grid too large (%lld row tiles, %lld batches x splits)",
-              (long long)gy, (long long)gz);
-  const dim3 grid((a.N + kF32B - 1) / kF32B, (unsigned)gy, (unsigned)gz);
-  const int es = dtype_in == LTV_DTYPE_BF16 ? 2 : 4;
-  const int la = f32m_stage(a.A, a.sam, a.sako, a.saki, a.sab, batches, a.kin, a.K, es);
-  const int lb = f32m_stage(a.B, a.sbn, a.sbko, a.sbki, a.sbb, batches, a.kin, a.K, es);
-  if (dtype_in == LTV_DTYPE_F32)
-    f32m_launch_ab<float, float>(la, lb, a, grid, st);
-  else if (dtype_out == LTV_DTYPE_BF16)
-    f32m_launch_ab<bf16_t, bf16_t>(la, lb, a, grid, st);
-  else
-    f32m_launch_ab<bf16_t, float>(la, lb, a, grid, st);
-  LTV_LAUNCH_CHECK();
-  return LTV_OK;
-}
-
 // Compute units of the current device (cached per device).
 int device_cu_count() {
   static int counts[64] = {0};
@@ -284,6 +214,60 @@ int device_cu_count() {
     counts[dev] = n;
   }
   return counts[dev];
+}
+
+// Whether the split GEMM takes 64 x 64 tiles: where 128 x 128 ones do not give
+// every CU a workgroup.  Measured on MI355X (128 / 64 tiles; both gradients
+// where two figures): fp32 B = 2, T = 300, K = 768, F = 2322 forward 41 / 27 us,
+// backward 170 / 91 us (108 and 36 large tiles); B = 1, T = 4097, K = 512,
+// F = 1040 backward 117 / 102 us (132); bf16 B = 9, T = 100 forward 15.5 / 10.8
+// us (81); above it they lose: fp32 B = 8, T = 1024, K = 768 backward 418 / 455
+// us (384).
+bool split_small(int M, int N, int batches) {
+  const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * batches;
+  return tiles < device_cu_count();
+}
+
+// C (dtype_out; fp32 for split partials) = A . B^T over `batches` batches and
+// `splits` reduction splits, on the split GEMM; LA, LB: which way each operand
+// is contiguous.
+template <int LA, int LB, int WB>
+int launch_split_wb(int dtype_in, int dtype_out, SplitArgs a, int batches, int splits,
+                    hipStream_t st) {
+  constexpr int R = 64 * WB;
+  const int bk = dtype_in == LTV_DTYPE_F32 ? SplitTraits<float>::bk(R) : SplitTraits<bf16_t>::bk(R);
+  const int64_t whole = (int64_t)a.KO * (a.kin / bk);
+  LTV_REQUIRE(whole < (1ll << 30), LTV_ERR_UNSUPPORTED, "split GEMM: reduction too long");
+  a.splits = std::max(1, splits);
+  a.split_whole = (int)((whole + a.splits - 1) / a.splits);
+  a.split_tail = (a.KO + a.splits - 1) / a.splits;
+  const int64_t gy = (a.M + R - 1) / R, gz = (int64_t)batches * a.splits;
+  LTV_REQUIRE(gy <= 65535 && gz <= 65535, LTV_ERR_UNSUPPORTED,
+              "split GEMM grid too large (%lld row tiles, %lld batches x splits)",
+              (long long)gy, (long long)gz);
+  const dim3 grid((a.N + R - 1) / R, (unsigned)gy, (unsigned)gz), blk(kSplitThreads);
+  if (dtype_in == LTV_DTYPE_F32)
+    hipLaunchKernelGGL((gemm_split_kernel<float, float, LA, LB, WB>), grid, blk, 0, st, a);
+  else if (dtype_out == LTV_DTYPE_BF16)
+    hipLaunchKernelGGL((gemm_split_kernel<bf16_t, bf16_t, LA, LB, WB>), grid, blk, 0, st, a);
+  else
+    hipLaunchKernelGGL((gemm_split_kernel<bf16_t, float, LA, LB, WB>), grid, blk, 0, st, a);
+  LTV_LAUNCH_CHECK();
+  return LTV_OK;
+}
+
+template <int LA, int LB>
+int launch_split(int dtype_in, int dtype_out, const SplitArgs& a, int batches, int splits,
+                 hipStream_t st) {
+  if (a.M == 0 || a.N == 0 || batches == 0) return LTV_OK;
+  LTV_REQUIRE((dtype_in == LTV_DTYPE_F32 && dtype_out == LTV_DTYPE_F32) ||
+                  (dtype_in == LTV_DTYPE_BF16 &&
+                   (dtype_out == LTV_DTYPE_BF16 || dtype_out == LTV_DTYPE_F32)),
+              LTV_ERR_UNSUPPORTED, "split GEMM: unsupported dtypes %d -> %d", dtype_in,
+              dtype_out);
+  if (splits <= 1 && split_small(a.M, a.N, batches))
+    return launch_split_wb<LA, LB, 1>(dtype_in, dtype_out, a, batches, splits, st);
+  return launch_split_wb<LA, LB, 2>(dtype_in, dtype_out, a, batches, splits, st);
 }
 
 // Persistent launch: one workgroup per compute unit (the tiles use most of the
@@ -409,12 +393,12 @@ extern "C" int ltv_linear_transpose_forward(int dtype, const void* x, const void
     }
   }
   // per batch: out_b (F x T) = W (F x K) . x_b^T
-  F32mArgs a{};
-  a.A = weight; a.sam = K; a.sako = 0; a.saki = 1; a.sab = 0;
-  a.B = x; a.sbn = K; a.sbko = 0; a.sbki = 1; a.sbb = (int64_t)T * K;
+  SplitArgs a{};
+  a.A = weight; a.sam = K; a.saki = 1;
+  a.B = x; a.sbn = K; a.sbki = 1; a.sbb = (int64_t)T * K;
   a.C = out; a.scm = T; a.scn = 1; a.scb = (int64_t)F * T;
-  a.M = F; a.N = T; a.K = K; a.kin = K > 0 ? K : 1;
-  return launch_f32m(dtype, dtype, a, B, 1, 0, st);
+  a.M = F; a.N = T; a.KO = K > 0 ? 1 : 0; a.kin = K;
+  return launch_split<kSplitKC, kSplitKC>(dtype, dtype, a, B, 1, st);
 }
 
 namespace {
@@ -441,18 +425,15 @@ LtSplits lt_splits(int M, int K, int F) {
   return p;
 }
 
-// grad_weight's split over the B T reduction on the fp32-MFMA GEMM.  With
-// `slots` workgroups resident at once (two per CU) and `tiles` 128 x 128
-// output tiles, S splits take ceil(tiles S / slots) rounds of M / S
-// reduction indices each: S minimises rounds / S (the smallest S within 4%
-// of the best, up to 32 splits of at least 256 indices).  At d12 (114 tiles,
-// 512 slots) S = 13: 1,482 items in 3 rounds (S = 5 leaves 58 items for a
-// second round, S = 4 a quarter of the slots idle).  S = 1 needs no workspace.
-LtSplits lt_f32m_splits(int M, int K, int F) {
-  LtSplits p;
-  p.Fr = F;
-  const int tiles = std::max(1, ((K + kF32B - 1) / kF32B) * ((F + kF32B - 1) / kF32B));
-  const int slots = 2 * device_cu_count();
+// grad_weight's split over the B T reduction on the split GEMM.  With `slots`
+// workgroups resident at once (kSplitWgPerCu per CU) and `tiles` 128 x 128
+// output tiles, S splits take ceil(tiles S / slots) rounds of 1 / S of the
+// reduction each: S minimises rounds / S (the smallest S within 4% of the best,
+// up to 32 splits of at least 256 indices).  S = 1 needs no workspace.
+int lt_split_splits(int B, int T, int K, int F) {
+  const int64_t M = (int64_t)B * T;
+  const int64_t tiles = std::max<int64_t>(1, (int64_t)((K + 127) / 128) * ((F + 127) / 128));
+  const int slots = kSplitWgPerCu * device_cu_count();
   auto cost = [&](int s) { return (double)((tiles * s + slots - 1) / slots) / s; };
   double best = cost(1);
   int smax = 1;
@@ -462,9 +443,7 @@ LtSplits lt_f32m_splits(int M, int K, int F) {
   }
   int S = 1;
   while (S < smax && cost(S) > 1.04 * best) ++S;
-  p.rows = std::max(kF32BK, round_up((M + S - 1) / S, kF32BK));
-  p.S = std::max(1, (M + p.rows - 1) / p.rows);
-  return p;
+  return S;
 }
 
 // Only tensors with no elements may be null (PyTorch hands those over as 0).
@@ -476,54 +455,59 @@ bool lt_backward_pointers_ok(const void* x, const void* weight, const void* grad
          (grad_weight || nw == 0) && (grad_out || ng == 0);
 }
 
-size_t lt_f32m_workspace(int B, int T, int K, int F) {
-  const LtSplits p = lt_f32m_splits(B * T, K, F);
-  return p.S > 1 ? (size_t)p.S * F * K * sizeof(float) : 0;
+size_t lt_split_workspace(int B, int T, int K, int F) {
+  const int S = lt_split_splits(B, T, K, F);
+  return S > 1 ? (size_t)S * F * K * sizeof(float) : 0;
 }
 
-// Both gradients on the fp32-MFMA GEMM.  grad_weight is split over the B T
+// Both gradients on the split GEMM.  grad_weight is split over the B T
 // reduction into fp32 partials in `workspace` when it holds
-// lt_f32m_workspace() bytes (then summed in a fixed order), else computed in
+// lt_split_workspace() bytes (then summed in a fixed order), else computed in
 // one pass per output tile.
-int lt_backward_f32m(int dtype, const void* x, const void* weight, const void* grad_out,
-                     int grad_out_is_btf, void* grad_x, void* grad_weight, void* workspace,
-                     size_t workspace_bytes, int B, int T, int K, int F, hipStream_t st) {
+int lt_backward_split(int dtype, const void* x, const void* weight, const void* grad_out,
+                      int grad_out_is_btf, void* grad_x, void* grad_weight, void* workspace,
+                      size_t workspace_bytes, int B, int T, int K, int F, hipStream_t st) {
   // grad_out element (b, f, t): (B,F,T) -> b*F*T + f*T + t ; (B,T,F) -> b*T*F + t*F + f
-  const int64_t go_f = grad_out_is_btf ? 1 : T;
-  const int64_t go_t = grad_out_is_btf ? F : 1;
+  const bool btf = grad_out_is_btf != 0;
+  const int64_t go_f = btf ? 1 : T;
+  const int64_t go_t = btf ? F : 1;
   // grad_x_b (T x K) = sum_f go_b(f, t) W(f, k)
-  F32mArgs a{};
-  a.A = grad_out; a.sam = go_t; a.sako = 0; a.saki = go_f; a.sab = (int64_t)F * T;
-  a.B = weight; a.sbn = 1; a.sbko = 0; a.sbki = K; a.sbb = 0;
+  SplitArgs a{};
+  a.A = grad_out; a.sam = go_t; a.saki = go_f; a.sab = (int64_t)F * T;
+  a.B = weight; a.sbn = 1; a.sbki = K;
   a.C = grad_x; a.scm = K; a.scn = 1; a.scb = (int64_t)T * K;
-  a.M = T; a.N = K; a.K = F; a.kin = F > 0 ? F : 1;
-  int rc = launch_f32m(dtype, dtype, a, B, 1, 0, st);
+  a.M = T; a.N = K; a.KO = F > 0 ? 1 : 0; a.kin = F;
+  int rc = btf ? launch_split<kSplitKC, kSplitRC>(dtype, dtype, a, B, 1, st)
+               : launch_split<kSplitRC, kSplitRC>(dtype, dtype, a, B, 1, st);
   if (rc) return rc;
-  // grad_W (F x K) = sum_{b,t} go(b, f, t) x(b, t, k); reduction index kk = b*T + t
+  // grad_W (F x K) = sum_{b,t} go(b, f, t) x(b, t, k): outer index b, inner t
   // (an empty reduction, B T = 0, stores zeros)
-  F32mArgs w{};
-  w.A = grad_out; w.sam = go_f; w.sako = (int64_t)F * T; w.saki = go_t; w.sab = 0;
-  w.B = x; w.sbn = 1; w.sbko = (int64_t)T * K; w.sbki = K; w.sbb = 0;
-  w.C = grad_weight; w.scm = K; w.scn = 1; w.scb = 0;
-  w.M = F; w.N = K; w.K = B * T; w.kin = T > 0 ? T : 1;
-  const LtSplits sp = lt_f32m_splits(w.K, K, F);
-  const size_t need = lt_f32m_workspace(B, T, K, F);
-  if (need == 0 || workspace == nullptr || workspace_bytes < need)
-    return launch_f32m(dtype, dtype, w, 1, 1, 0, st);
+  SplitArgs w{};
+  w.A = grad_out; w.sam = go_f; w.sako = (int64_t)F * T; w.saki = go_t;
+  w.B = x; w.sbn = 1; w.sbko = (int64_t)T * K; w.sbki = K;
+  w.C = grad_weight; w.scm = K; w.scn = 1;
+  w.M = F; w.N = K; w.KO = T > 0 ? B : 0; w.kin = T;
+  auto launch_w = [&](int dtype_out, int S) {
+    return btf ? launch_split<kSplitRC, kSplitRC>(dtype, dtype_out, w, 1, S, st)
+               : launch_split<kSplitKC, kSplitRC>(dtype, dtype_out, w, 1, S, st);
+  };
+  const int S = lt_split_splits(B, T, K, F);
+  const size_t need = lt_split_workspace(B, T, K, F);
+  if (need == 0 || workspace == nullptr || workspace_bytes < need) return launch_w(dtype, 1);
   w.C = workspace;
   w.scs = (int64_t)F * K;
-  rc = launch_f32m(dtype, LTV_DTYPE_F32, w, 1, sp.S, sp.rows, st);
+  rc = launch_w(LTV_DTYPE_F32, S);
   if (rc) return rc;
   const int64_t n = (int64_t)F * K;
   const int blocks = (int)std::min<int64_t>((n + 255) / 256, 8192);
   if (dtype == LTV_DTYPE_F32)
     hipLaunchKernelGGL(reduce_splits_kernel<float>, dim3(blocks), dim3(256), 0, st,
                        reinterpret_cast<const float*>(workspace),
-                       reinterpret_cast<float*>(grad_weight), sp.S, n, n);
+                       reinterpret_cast<float*>(grad_weight), S, n, n);
   else
     hipLaunchKernelGGL(reduce_splits_kernel<bf16_t>, dim3(blocks), dim3(256), 0, st,
                        reinterpret_cast<const float*>(workspace),
-                       reinterpret_cast<bf16_t*>(grad_weight), sp.S, n, n);
+                       reinterpret_cast<bf16_t*>(grad_weight), S, n, n);
   LTV_LAUNCH_CHECK();
   return LTV_OK;
 }
@@ -538,14 +522,14 @@ extern "C" int ltv_linear_transpose_backward(int dtype, const void* x, const voi
   LTV_REQUIRE(B >= 0 && T >= 0 && K >= 0 && F >= 0, LTV_ERR_INVALID_ARG, "negative size");
   LTV_REQUIRE(lt_backward_pointers_ok(x, weight, grad_out, grad_x, grad_weight, B, T, K, F),
               LTV_ERR_INVALID_ARG, "null tensor pointer");
-  return lt_backward_f32m(dtype, x, weight, grad_out, grad_out_is_btf, grad_x, grad_weight,
+  return lt_backward_split(dtype, x, weight, grad_out, grad_out_is_btf, grad_x, grad_weight,
                           nullptr, 0, B, T, K, F, (hipStream_t)stream);
 }
 
 extern "C" size_t ltv_linear_transpose_backward_workspace_size(int dtype, int B, int T, int K,
                                                                 int F, int grad_out_is_btf) {
   if (B <= 0 || T <= 0 || K <= 0 || F <= 0) return 0;
-  if (!lt_backward_mfma(dtype, grad_out_is_btf, B, T, K, F)) return lt_f32m_workspace(B, T, K, F);
+  if (!lt_backward_mfma(dtype, grad_out_is_btf, B, T, K, F)) return lt_split_workspace(B, T, K, F);
   const LtSplits p = lt_splits(B * T, K, F);
   return (size_t)p.S * p.Fr * K * sizeof(float);
 }
@@ -564,7 +548,7 @@ extern "C" int ltv_linear_transpose_backward_ws(int dtype, const void* x, const 
   if (!lt_backward_mfma(dtype, grad_out_is_btf, B, T, K, F) ||
       !(aligned16(x) && aligned16(weight) && aligned16(grad_out) && aligned16(grad_x) &&
         aligned16(grad_weight)))
-    return lt_backward_f32m(dtype, x, weight, grad_out, grad_out_is_btf, grad_x, grad_weight,
+    return lt_backward_split(dtype, x, weight, grad_out, grad_out_is_btf, grad_x, grad_weight,
                             workspace, workspace_bytes, B, T, K, F, st);
   const int M = B * T;
   const LtSplits sp = lt_splits(M, K, F);

@@ -1,0 +1,524 @@
+// bf16-MFMA GEMM over strided operands of any alignment, in fp32 and bf16
+// (gfx950 v_mfma_f32_32x32x16_bf16, fp32 sums): the engine of the
+// reference-layout fused_linear_transpose op in fp32, and in bf16 for the
+// layouts the direct-to-LDS kernels do not take (a time axis that is not a
+// multiple of their tile, operands that start off a 16-byte boundary).
+//
+//   C(m, n) = sum_{ko < KO} sum_{ki < kin} A(m, ko, ki) B(n, ko, ki)
+//   A(m, ko, ki) at A + m sam + ko sako + ki saki (+ z sab for batch z), B alike
+//
+// fp32 operands are split exactly into three bf16 pieces, x = x1 + x2 + x3 (each
+// the rest rounded to nearest: 8 + 8 + 8 bits of the significand), and a
+// product is six MFMA terms, smallest first: x3 y1, x1 y3, x2 y2, x2 y1, x1 y2,
+// x1 y1.  The three left out are below 2^-26 of the product -- under the rounding
+// of one fp32 addition (2^-24 of the sum) that every partial sum takes anyway.
+// A bf16 MFMA term is 16 times as fast as the fp32 MFMA (2.5 against 0.157
+// PFLOP/s nominal), six of them 2.7 times.  Non-finite results send the
+// wavefront's part of the tile through the fp32 MFMA instead (an infinity has
+// no such split, nor has a value that rounds past the largest bf16), so
+// infinities and NaNs come out as fp32 arithmetic gives them.
+// bf16 operands are one piece: the products are exact, as they always were.
+//
+// Measured on MI355X against the fp32-MFMA kernel before it (128 x 128 tiles,
+// quads, one element per load off a 16-byte boundary), 2-norm errors against
+// float64:
+//   fp32 B = 32, T = 1024, K = 768, F = 2322: forward 1070 -> 712 us (164
+//     TFLOP/s), both gradients 2030 -> 1256 us (186); errors 5.0e-7 -> 4.2e-7
+//     (forward), 8.6e-7 -> 7.5e-7 (grad_x), 9.0e-7 -> 9.1e-7 (grad_weight);
+//   fp32 B = 8: 309 -> 197 and 645 -> 405 us; B = 2, T = 300: 58 -> 27, 214 -> 83;
+//   bf16 B = 20, T = 1501, K = 768, F = 2322: 971 -> 194 us (551 TFLOP/s), 3265
+//     -> 408 us (524); B = 5, T = 1501, K = 512, F = 1040: 117 -> 25, 328 -> 75.
+// What bounds the fp32 form: the matrix cores are busy 65% of the cycles (32
+// per MFMA, counted) at the clock that random operands leave; halving the
+// conversion's instructions gained 3%.
+//
+// 128 x 128 output tiles, 4 wavefronts of 64 x 64, three workgroups per CU
+// (three wavefronts per SIMD, so that one's barrier, load wait or conversion
+// leaves the matrix core to the others); 64 x 64 tiles where those are too few.
+// The global loads run two steps ahead in registers, and the next step is
+// converted into the other of two LDS stages while this one runs its MFMAs; one
+// barrier per step.
+//
+// An operand must be contiguous along its reduction (kSplitKC) or its rows
+// (kSplitRC).  A thread loads chunks of 8 consecutive elements -- aligned
+// to an element only: an odd bf16 chunk is read as whole dwords and shifted --
+// and writes them to LDS as 16-byte chunks in the operand's own orientation:
+//   KC  [row][k]: chunk c of row r at slot c ^ ((r / phase) & (chunks - 1)), phase
+//       the rows of a 256-byte bank window, read with ds_read_b128;
+//   RC  [k][row]: row-chunk c of k-row k at slot c ^ (4 (k & 3)), read with
+//       ds_read_b64_tr_b16;
+// both fragment reads are then free of bank conflicts.
+//
+// Steps never straddle an outer index: each ko has kin / BK whole steps and, where
+// kin is not a multiple, a last one padded with zeros.  A workgroup runs its
+// whole steps first, pipelined, then the partial ones.  Split-K: blockIdx.z =
+// batch * splits + split; split s takes the whole steps [s split_whole,
+// (s + 1) split_whole) and the partial ones of the outer indices [s split_tail,
+// (s + 1) split_tail), and sums them into C + s scs.
+#pragma once
+
+#include "ltv_gemm_dma.hpp"
+
+namespace ltv {
+
+enum SplitLayout { kSplitKC = 0, kSplitRC = 1 };
+
+constexpr int kSplitThreads = 256;  // 4 wavefronts, 2 x 2
+constexpr int kSplitWgPerCu = 3;
+
+// Pieces per element, and the k-step of a tile of R = 128 or 64 rows.
+template <typename TI>
+struct SplitTraits {
+  static constexpr int kPieces = sizeof(TI) == 4 ? 3 : 1;
+  __host__ __device__ static constexpr int bk(int R) { return sizeof(TI) == 4 && R == 128 ? 16 : 32; }
+};
+
+struct SplitArgs {
+  const void* A;
+  int64_t sam, sako, saki, sab;
+  const void* B;
+  int64_t sbn, sbko, sbki, sbb;
+  void* C;
+  int64_t scm, scn, scb, scs;  // output strides: row, column, batch, split
+  int M, N, KO, kin;
+  int split_whole;  // whole k-steps (of the KO (kin / BK)) per split
+  int split_tail;   // outer indices whose last, partial step a split takes
+  int splits;
+};
+
+// One operand of one workgroup: its rows [row0, row0 + 128).
+template <typename TI>
+struct SplitOperand {
+  const TI* p;  // at the workgroup's batch
+  int64_t sr, sko, ski;
+  int rows, kin, row0;
+  bool odd;  // bf16: some chunk may start inside a dword
+};
+
+typedef uint32_t u32x4a4_t __attribute__((ext_vector_type(4), aligned(4)));
+
+// A thread's chunks of one operand tile, as loaded.
+template <typename TI, int R>
+struct SplitRaw {
+  static constexpr int BK = SplitTraits<TI>::bk(R);
+  static constexpr int NC = R * BK / 8 / kSplitThreads;  // chunks per thread
+  static constexpr int W = sizeof(TI) == 4 ? 8 : 5;  // dwords (bf16: one more, for odd starts)
+  static_assert(NC >= 1 && NC * 8 * kSplitThreads == R * BK, "whole chunks per thread");
+  uint32_t w[NC][W];
+};
+
+// Global -> registers -> LDS staging of one R-row x BK tile.
+template <typename TI, int L, int R>
+struct SplitStager {
+  using Raw = SplitRaw<TI, R>;
+  static constexpr int E = sizeof(TI);
+  static constexpr int BK = Raw::BK, NP = SplitTraits<TI>::kPieces, NC = Raw::NC;
+  static constexpr int CPR = BK / 8;           // chunks per KC row
+  static constexpr int kPlane = R * BK * 2;    // bytes of one piece's plane
+
+  // chunk c at ko = 0, k0 = 0.  Rows past the operand: row 0.  An RC chunk that
+  // the operand's end cuts is read `early` rows early, to end with it, and
+  // shifted into place when it is stored.
+  const TI* rp[NC];
+  uint32_t early;
+
+  // row (KC) or first row (RC), and k within the step, of chunk c
+  __device__ __forceinline__ static int row_of(int c) {
+    const int q = threadIdx.x + kSplitThreads * c;
+    return L == kSplitKC ? q / CPR : 8 * (q % (R / 8));
+  }
+  __device__ __forceinline__ static int k_of(int c) {
+    const int q = threadIdx.x + kSplitThreads * c;
+    return L == kSplitKC ? 8 * (q % CPR) : q / (R / 8);
+  }
+
+  __device__ __forceinline__ void setup(const SplitOperand<TI>& op) {
+    // (an RC thread's chunks share their rows)
+    const int over = op.row0 + row_of(0) + 8 - op.rows;
+    early = L == kSplitRC && over > 0 && over < 8 ? (uint32_t)over : 0u;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int row = op.row0 + row_of(c);
+      const int64_t r = row < op.rows ? row - (int)early : 0;
+      rp[c] = L == kSplitKC ? op.p + r * op.sr + k_of(c) : op.p + r + (int64_t)k_of(c) * op.ski;
+    }
+  }
+
+  // 8 elements from p (aligned to an element)
+  __device__ __forceinline__ static void load_chunk(Raw& o, int c, const TI* p, bool odd) {
+    if constexpr (E == 4) {
+      const u32x4a4_t a = *reinterpret_cast<const u32x4a4_t*>(p);
+      const u32x4a4_t b = *reinterpret_cast<const u32x4a4_t*>(p + 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        o.w[c][i] = a[i];
+        o.w[c][4 + i] = b[i];
+      }
+    } else {
+      const uintptr_t a = reinterpret_cast<uintptr_t>(p);
+      const uint32_t* q = reinterpret_cast<const uint32_t*>(a & ~(uintptr_t)3);
+      const u32x4a4_t v = *reinterpret_cast<const u32x4a4_t*>(q);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o.w[c][i] = v[i];
+      if (odd) {
+        // an odd chunk ends in the next dword; an even one reads no further
+        o.w[c][4] = q[(a & 2u) != 0 ? 4 : 0];
+      }
+    }
+  }
+
+  // A step inside the reduction: off elements from the first one.
+  __device__ __forceinline__ void load(Raw& o, const SplitOperand<TI>& op, int64_t off) const {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) load_chunk(o, c, rp[c] + off, op.odd);
+  }
+
+  // Any step, element by element, to chunks that start on a dword.
+  __device__ __forceinline__ void load_checked(Raw& o, const SplitOperand<TI>& op, int64_t off,
+                                               int k0) const {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      // valid elements of the chunk, from its first on
+      const int row = op.row0 + row_of(c), k = k0 + k_of(c);
+      int n = L == kSplitKC ? (row < op.rows ? op.kin - k : 0) : (k < op.kin ? op.rows - row : 0);
+      n = n < 0 ? 0 : n > 8 ? 8 : n;
+#pragma unroll
+      for (int i = 0; i < Raw::W; ++i) o.w[c][i] = 0u;
+      const TI* p = rp[c] + off + early;
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (e < n) {
+          if constexpr (E == 4)
+            o.w[c][e] = __float_as_uint(p[e]);
+          else
+            o.w[c][e >> 1] |= (uint32_t)p[e] << (16 * (e & 1));
+        }
+    }
+  }
+
+  // The chunks as bf16 pieces to the planes at lds.  CHECKED: from
+  // load_checked; else from load at the same `off`.
+  template <bool CHECKED>
+  __device__ __forceinline__ void store(Raw& o, char* lds, const SplitOperand<TI>& op,
+                                        int64_t off) const {
+    const bool cut = !CHECKED && L == kSplitRC && op.row0 + R > op.rows && op.rows % 8 != 0;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int r = row_of(c), k = k_of(c);
+      // (rows past the operand hold row 0 or zeros: their results are not stored)
+      uint32_t at;
+      if (L == kSplitKC) {
+        constexpr int kRow = BK * 2, kPhase = 256 / kRow;
+        at = (uint32_t)(r * kRow + (((k >> 3) ^ ((r / kPhase) & (CPR - 1))) << 4));
+      } else {
+        at = (uint32_t)(k * (R * 2) + (((r >> 3) ^ rc_swizzle(k)) << 4));
+      }
+      uint4* d = reinterpret_cast<uint4*>(lds + at);
+      if constexpr (E == 2) {
+        if (!CHECKED && op.odd) {
+          const uint32_t sh = (uint32_t)(reinterpret_cast<uintptr_t>(rp[c] + off) & 2u) << 3;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            o.w[c][i] = __builtin_amdgcn_alignbit(o.w[c][i + 1], o.w[c][i], sh);
+        }
+        if (cut) shift_down<4, 2>(o.w[c], early);
+        d[0] = make_uint4(o.w[c][0], o.w[c][1], o.w[c][2], o.w[c][3]);
+      } else {
+        if (cut) shift_down<8, 1>(o.w[c], early);
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = __uint_as_float(o.w[c][e]);
+        static_for<NP>([&](auto pc) {
+          constexpr int p = decltype(pc)::value;
+          uint32_t q[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            q[i] = cvt_pk_bf16(x[2 * i], x[2 * i + 1]);
+            if (p + 1 < NP) {
+              // the rest, exact: x - (1, 0) . q and x - (0, 1) . q
+              x[2 * i] = rest(q[i], 0x0000bf80u, x[2 * i]);
+              x[2 * i + 1] = rest(q[i], 0xbf800000u, x[2 * i + 1]);
+            }
+          }
+          d[p * (kPlane / 16)] = make_uint4(q[0], q[1], q[2], q[3]);
+        });
+      }
+    }
+  }
+
+  // x + q . m for a pair of bf16 q and m = (-1, 0) or (0, -1): one instruction
+  // (v_dot2_f32_bf16) where widening q and subtracting takes two.  m goes through
+  // a register: the pair (-1, 0) written as the instruction's inline -1.0 measured
+  // as (0, -1).
+  __device__ __forceinline__ static float rest(uint32_t q, uint32_t m, float x) {
+    asm("" : "+s"(m));
+    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, q),
+                                           __builtin_bit_cast(bf16x2_t, m), x, false);
+  }
+
+  // The first N dwords of w (EPD elements each) moved down by n < 8 elements,
+  // zeros following.
+  template <int N, int EPD>
+  __device__ __forceinline__ static void shift_down(uint32_t (&w)[Raw::W], uint32_t n) {
+    if (EPD == 2) {
+      const uint32_t sh = 16u * (n & 1u);
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        w[i] = __builtin_amdgcn_alignbit(i + 1 < N ? w[i + 1] : 0u, w[i], sh);
+    }
+    const uint32_t m = n / EPD;
+    static_for<3>([&](auto lc) {
+      constexpr int step = 1 << decltype(lc)::value;
+      if constexpr (step < N) {
+        const bool on = (m & step) != 0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) w[i] = on ? (i + step < N ? w[i + step] : 0u) : w[i];
+      }
+    });
+  }
+
+  // Slot swizzle of k-row k of an RC tile: the four k-rows one 16-lane group of
+  // ds_read_b64_tr_b16 reads land in four disjoint 64-byte windows (rows of
+  // 256 bytes, or two to the 256-byte bank window).
+  __device__ __forceinline__ static int rc_swizzle(int k) {
+    return R == 128 ? 4 * (k & 3) : 4 * ((k >> 1) & 1);
+  }
+
+  // MFMA operand fragment (8 consecutive k of row rb + lane % 32) of k16 sub-step t.
+  __device__ __forceinline__ static bf16x8_t frag(const char* plane, int rb, int t, int lane) {
+    typedef __attribute__((address_space(3))) const char lds_char;
+    lds_char* base = (lds_char*)plane;
+    if (L == kSplitRC) {
+      const int g = lane >> 4, s = lane & 15;
+      const int row = rb + (g & 1) * 16 + 4 * (s & 3);
+      const int k = t * 16 + (g >> 1) * 8 + (s >> 2);
+      typedef __attribute__((address_space(3))) i16x4_t lds_i16x4;
+      lds_char* p0 = base + k * (R * 2) + (((row >> 3) ^ rc_swizzle(k)) << 4) + (row & 7) * 2;
+      lds_char* p1 = p0 + 4 * (R * 2);  // k + 4: the same swizzle
+      const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)p0);
+      const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)p1);
+      typedef short i16x8_t __attribute__((ext_vector_type(8)));
+      const i16x8_t v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      return __builtin_bit_cast(bf16x8_t, v);
+    }
+    constexpr int kRow = BK * 2, kPhase = 256 / kRow;
+    const int r = rb + (lane & 31), c = 2 * t + (lane >> 5);
+    return __builtin_bit_cast(
+        bf16x8_t, *(__attribute__((address_space(3))) const u32x4_t*)(
+                      base + r * kRow + ((c ^ ((r / kPhase) & (CPR - 1))) << 4)));
+  }
+};
+
+// One k-step [k0, k1) of outer index ko of the 32 x 32 block of A rows m0..,
+// B rows n0.., on the fp32 MFMA straight from memory: only for results that
+// are not finite.
+__device__ __forceinline__ void split_block_f32(const SplitOperand<float>& a,
+                                                const SplitOperand<float>& b, int m0, int n0,
+                                                int ko, int k0, int k1, int lane,
+                                                f32x16_t& acc) {
+  const int m = m0 + (lane & 31), n = n0 + (lane & 31);
+  for (int kk = k0; kk < k1; kk += 2) {
+    const int k = kk + (lane >> 5);
+    float x = 0.0f, y = 0.0f;
+    if (k < k1 && m < a.rows) x = a.p[m * a.sr + ko * a.sko + k * a.ski];
+    if (k < k1 && n < b.rows) y = b.p[n * b.sr + ko * b.sko + k * b.ski];
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc, 0, 0, 0);
+  }
+}
+
+// WB x WB blocks of 32 x 32 per wavefront: tiles of R = 64 WB rows of A and of B.
+template <typename TI, typename TO, int LA, int LB, int WB>
+__global__ void __launch_bounds__(kSplitThreads, kSplitWgPerCu)
+gemm_split_kernel(const SplitArgs g) {
+  constexpr int R = 64 * WB;
+  using StA = SplitStager<TI, LA, R>;
+  using StB = SplitStager<TI, LB, R>;
+  constexpr int BK = StA::BK, NP = StA::NP, kPlane = StA::kPlane;
+  __shared__ __attribute__((aligned(1024))) char lds_a[2][NP * kPlane];
+  __shared__ __attribute__((aligned(1024))) char lds_b[2][NP * kPlane];
+
+  // workgroup w (dispatch order) runs on XCD w % 8: deal the tiles to the XCDs
+  // in contiguous ranges (n-tiles fastest), so tiles sharing an operand tile
+  // share that XCD's L2.  XCD x holds the workgroups x, x + 8, ... < total:
+  // q + (x < r) of them (q, r = total / 8, total % 8), tiles from x q + min(x, r).
+  const int gx = gridDim.x, gy = gridDim.y;
+  const int64_t total = (int64_t)gx * gy * gridDim.z;
+  const int64_t wg = blockIdx.x + (int64_t)gx * (blockIdx.y + (int64_t)gy * blockIdx.z);
+  const int64_t xcd = wg % 8, q = total / 8, r = total % 8;
+  const int64_t u = xcd * q + (xcd < r ? xcd : r) + wg / 8;
+  const int tx = (int)(u % gx), ty = (int)((u / gx) % gy), z = (int)(u / ((int64_t)gx * gy));
+  const int batch = z / g.splits, split = z - batch * g.splits;
+  const int m0 = ty * R, n0 = tx * R;
+
+  auto odd = [](const void* p, int64_t a, int64_t b, int64_t c) {
+    return sizeof(TI) == 2 && (((reinterpret_cast<uintptr_t>(p) >> 1) | a | b | c) & 1) != 0;
+  };
+  const SplitOperand<TI> oa{reinterpret_cast<const TI*>(g.A) + (int64_t)batch * g.sab, g.sam,
+                            g.sako, g.saki, g.M, g.kin, m0,
+                            odd(g.A, g.sab, g.sako, LA == kSplitKC ? g.sam : g.saki | g.M)};
+  const SplitOperand<TI> ob{reinterpret_cast<const TI*>(g.B) + (int64_t)batch * g.sbb, g.sbn,
+                            g.sbko, g.sbki, g.N, g.kin, n0,
+                            odd(g.B, g.sbb, g.sbko, LB == kSplitKC ? g.sbn : g.sbki | g.N)};
+
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int wm = (wave & 1) * (32 * WB), wn = (wave >> 1) * (32 * WB);
+
+  f32x16_t acc[WB][WB];
+#pragma unroll
+  for (int a = 0; a < WB; ++a)
+#pragma unroll
+    for (int b = 0; b < WB; ++b)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
+
+  StA sa;
+  StB sb;
+  sa.setup(oa);
+  sb.setup(ob);
+  auto mfmas = [&](int cur) {
+#pragma unroll
+    for (int t = 0; t < BK / 16; ++t) {
+      bf16x8_t fa[NP][WB], fb[NP][WB];
+#pragma unroll
+      for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int a = 0; a < WB; ++a) {
+          fa[p][a] = StA::frag(lds_a[cur] + p * kPlane, wm + 32 * a, t, lane);
+          fb[p][a] = StB::frag(lds_b[cur] + p * kPlane, wn + 32 * a, t, lane);
+        }
+      auto term = [&](int pa, int pb) {
+#pragma unroll
+        for (int a = 0; a < WB; ++a)
+#pragma unroll
+          for (int b = 0; b < WB; ++b)
+            acc[a][b] =
+                __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[pa][a], fb[pb][b], acc[a][b], 0, 0, 0);
+      };
+      if constexpr (NP == 3) {
+        term(2, 0);
+        term(0, 2);
+        term(1, 1);
+        term(1, 0);
+        term(0, 1);
+      }
+      term(0, 0);
+    }
+  };
+  SplitRaw<TI, R> ra[2], rb[2];
+
+  // The whole steps, an even number of them, pipelined: while step s runs, step
+  // s + 1 (loaded a step earlier) is converted and written to the other stage
+  // and step s + 2 is loaded, so a load has two steps to arrive.  Past the end
+  // the last step is loaded and stored again, unused: no branch in the loop.
+  const int wpb = g.kin / BK;  // whole steps per outer index
+  const int w0 = split * g.split_whole, w1 = min(g.KO * wpb, w0 + g.split_whole);
+  const bool rows_ok = (LA != kSplitRC || g.M >= 8) && (LB != kSplitRC || g.N >= 8);
+  const int np = rows_ok && w1 > w0 ? (w1 - w0) & ~1 : 0;
+  if (np > 0) {
+    int ko = w0 / wpb, ki = w0 - ko * wpb, left = np;
+    int64_t offa[2], offb[2];
+    auto load = [&](auto setc) {
+      constexpr int set = decltype(setc)::value;
+      offa[set] = (int64_t)ko * oa.sko + (int64_t)(ki * BK) * oa.ski;
+      offb[set] = (int64_t)ko * ob.sko + (int64_t)(ki * BK) * ob.ski;
+      sa.load(ra[set], oa, offa[set]);
+      sb.load(rb[set], ob, offb[set]);
+      const int nki = ki + 1 < wpb ? ki + 1 : 0, nko = ki + 1 < wpb ? ko : ko + 1;
+      --left;
+      ki = left > 0 ? nki : ki;
+      ko = left > 0 ? nko : ko;
+    };
+    auto store = [&](auto setc) {
+      constexpr int set = decltype(setc)::value;
+      sa.template store<false>(ra[set], lds_a[set], oa, offa[set]);
+      sb.template store<false>(rb[set], lds_b[set], ob, offb[set]);
+    };
+    using S0 = std::integral_constant<int, 0>;
+    using S1 = std::integral_constant<int, 1>;
+    load(S0{});
+    load(S1{});
+    store(S0{});
+    __syncthreads();
+    for (int s = 0; s < np; s += 2) {
+      // (a stage is refilled after the barrier that ended its last reads)
+      load(S0{});
+      mfmas(0);
+      store(S1{});
+      __syncthreads();
+      load(S1{});
+      mfmas(1);
+      store(S0{});
+      __syncthreads();
+    }
+  }
+  // The steps left: an odd whole one, and the ends of the outer indices' ranges
+  // (all of them where an RC operand has fewer rows than a chunk).
+  auto checked = [&](int ko, int k0) {
+    const int64_t fa = (int64_t)ko * oa.sko + (int64_t)k0 * oa.ski;
+    const int64_t fb = (int64_t)ko * ob.sko + (int64_t)k0 * ob.ski;
+    sa.load_checked(ra[0], oa, fa, k0);
+    sb.load_checked(rb[0], ob, fb, k0);
+    sa.template store<true>(ra[0], lds_a[0], oa, fa);
+    sb.template store<true>(rb[0], lds_b[0], ob, fb);
+    __syncthreads();
+    mfmas(0);
+    __syncthreads();
+  };
+  const int tails = wpb * BK < g.kin ? g.KO : 0;
+  const int t0 = split * g.split_tail, t1 = min(tails, t0 + g.split_tail);
+  const int nodd = w1 - w0 - np, ntail = t1 - t0;
+  for (int s = 0; s < (nodd > 0 ? nodd : 0) + (ntail > 0 ? ntail : 0); ++s) {
+    const bool whole = s < nodd;
+    const int w = w0 + np + s;
+    const int ko = whole ? w / wpb : t0 + s - (nodd > 0 ? nodd : 0);
+    checked(ko, whole ? (w - ko * wpb) * BK : wpb * BK);
+  }
+
+  if constexpr (NP == 3) {
+    bool bad = false;
+#pragma unroll
+    for (int a = 0; a < WB; ++a)
+#pragma unroll
+      for (int b = 0; b < WB; ++b)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) bad = bad || !(fabsf(acc[a][b][v]) < INFINITY);
+    if (__any(bad)) {
+#pragma unroll
+      for (int a = 0; a < WB; ++a)
+#pragma unroll
+        for (int b = 0; b < WB; ++b) {
+          f32x16_t c;
+#pragma unroll
+          for (int v = 0; v < 16; ++v) c[v] = 0.0f;
+          const int mb = m0 + wm + 32 * a, nb = n0 + wn + 32 * b;
+          for (int w = w0; w < w1; ++w) {
+            const int ko = w / wpb, k = (w - ko * wpb) * BK;
+            split_block_f32(oa, ob, mb, nb, ko, k, k + BK, lane, c);
+          }
+          for (int ko = t0; ko < t1; ++ko)
+            split_block_f32(oa, ob, mb, nb, ko, wpb * BK, g.kin, lane, c);
+          acc[a][b] = c;
+        }
+    }
+  }
+
+  // lane l of block (a, b) holds column n = 32 b + l % 32 and rows
+  // m = 32 a + 8 (v / 4) + 4 (l / 32) + v % 4
+  TO* C = reinterpret_cast<TO*>(g.C) + (int64_t)batch * g.scb + (int64_t)split * g.scs;
+#pragma unroll
+  for (int a = 0; a < WB; ++a)
+#pragma unroll
+    for (int b = 0; b < WB; ++b) {
+      const int n = n0 + wn + 32 * b + (lane & 31);
+      if (n >= g.N) continue;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int m = m0 + wm + 32 * a + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+        if (m < g.M) io_traits<TO>::store(C + (int64_t)m * g.scm + (int64_t)n * g.scn, acc[a][b][v]);
+      }
+    }
+}
+
+}  // namespace ltv

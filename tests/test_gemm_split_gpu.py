@@ -1,0 +1,74 @@
+"""The strided bf16-MFMA GEMM behind ``fused_linear_transpose``: fp32 operands
+as three bf16 pieces each, bf16 operands of any alignment.
+
+Sizes where it can go wrong: reductions of no, one, an even and an odd number of
+whole k-steps (16 or 32 indices) with and without a partial one, rows cut inside
+a chunk of 8 (fewer than 8, one past, one short of a chunk and of a tile), odd
+row pitches, both tile sizes (128 x 128 where those fill the device), several
+reduction splits.  Bounds: the worst case of an fp32 sum, as for the op.
+Infinities, NaNs and values past the largest bf16 come out as fp32 arithmetic
+gives them.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from test_linear_transpose_f32_gpu import DEV, _check, _operands, _ops
+
+pytestmark = pytest.mark.gpu
+DTYPES = [torch.float32, torch.bfloat16]
+
+
+def _run(B, T, K, F, dtype, btf, seed=0):
+    ops = _ops().nanochat_cuda
+    x, w, go = _operands(B, T, K, F, dtype, seed)
+    if btf:
+        go = go.transpose(1, 2).contiguous().transpose(1, 2)
+    bf = dtype == torch.bfloat16
+    case = f"B={B} T={T} K={K} F={F} {dtype} btf={btf}"
+    out = ops.fused_linear_transpose_cuda_op(x, w)
+    gx, gw = torch.empty_like(x), torch.empty_like(w)
+    ops.fused_linear_transpose_backward_kernel(x, w, go, gx, gw)
+    _check(out, w.unsqueeze(0).expand(B, F, K), x.transpose(1, 2), K, "out " + case, bf)
+    _check(gx, go.transpose(1, 2), w.unsqueeze(0).expand(B, F, K), F, "grad_x " + case, bf)
+    _check(gw, go.permute(1, 0, 2).reshape(F, B * T), x.reshape(B * T, K), B * T + 32,
+           "grad_weight " + case, bf)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "bf16"])
+@pytest.mark.parametrize("btf", [False, True], ids=["bft", "btf"])
+@pytest.mark.parametrize("K,F", [(8, 16), (15, 31), (16, 47), (33, 64), (71, 129), (128, 97)])
+def test_small_tiles(dtype, btf, K, F):
+    for T in (3, 7, 9, 16, 31, 33, 65, 127, 135):
+        _run(2, T, K, F, dtype, btf, seed=T)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "bf16"])
+@pytest.mark.parametrize("btf", [False, True], ids=["bft", "btf"])
+@pytest.mark.parametrize("T,K,F", [(129, 100, 333), (257, 72, 1041), (1000, 129, 161)])
+def test_large_tiles_and_splits(dtype, btf, T, K, F):
+    _run(40, T, K, F, dtype, btf, seed=T)
+
+
+@pytest.mark.parametrize("T", [40, 1024])
+def test_f32_non_finite(T):
+    """Every element of the result that an infinity, a NaN or a value past the
+    largest bf16 takes part in equals the fp32 arithmetic's class; the others
+    stay within the bound."""
+    B, K, F = 8, 96, 200
+    x, w, _ = _operands(B, T, K, F, torch.float32, 5)
+    big = 3.4e38  # rounds to infinity in bf16
+    x[0, 3, 5], x[1, 0, 0], x[2, 7, 95], x[3, 1, 2] = float("inf"), float("nan"), -float("inf"), big
+    w[17] = w[17].abs() * 2.0 ** -10  # positive: one sign per product with x[0, 3, 5]
+    w[18] = 0.0                        # 0 * inf
+    out = _ops().nanochat_cuda.fused_linear_transpose_cuda_op(x, w)
+    want = torch.matmul(w.double().unsqueeze(0), x.double().transpose(1, 2))
+    assert torch.equal(torch.isnan(out), torch.isnan(want))
+    inf = torch.isinf(want)
+    assert bool(inf.any()) and torch.equal(out.double()[inf], want[inf])
+    fin = torch.isfinite(want)
+    mag = torch.matmul(w.double().abs().unsqueeze(0), x.double().abs().transpose(1, 2))
+    assert bool(((out.double() - want).abs()[fin] <= (K + 4) * 2.0 ** -24 * mag[fin]).all())
+    assert float(out[3, 17, 1]) > 1e30
