@@ -198,64 +198,75 @@ int scan_launch_lb_channel(bool bf16, const BwdArgs& a, float* dalpha, float* du
   return LTV_OK;
 }
 
-// carry[bh, k, c] = g entering chunk k from its end: the maps of the
-// sub-chunks after chunk k applied to 0, last to first.  One thread per
-// (b h, channel); the maps are read in batches so the walk is not one load
-// latency per sub-chunk.
-__global__ void __launch_bounds__(256) scan_bwd_carry_kernel(const BwdArgs args) {
+// carry[bh, k, c] = g entering chunk k from its end: the maps of the chunks
+// after chunk k applied to 0, last to first.  One thread per (b h, channel);
+// the maps are read in batches so the walk is not one load latency per chunk.
+__global__ void __launch_bounds__(128) scan_bwd_carry_kernel(const BwdArgs args) {
   const ScanShape& S = args.sh;
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= (int64_t)S.B * S.H * S.D) return;
   const int c = (int)(idx % S.D);
   const int64_t bh = idx / S.D;
-  const int64_t plane = (int64_t)S.B * S.H * args.nfine * S.D;
-  const int fpc = args.chunk_steps / args.fine_steps;  // sub-chunks per chunk
-  const float* ap = args.agg + bh * args.nfine * S.D + c;
+  const int64_t plane = (int64_t)S.B * S.H * args.nchunk * S.D;
+  const float* ap = args.agg + bh * args.nchunk * S.D + c;
   float* cp = args.carry + bh * args.nchunk * S.D + c;
-  cp[(int64_t)(args.nchunk - 1) * S.D] = 0.0f;
   float g = 0.0f;
+  cp[(int64_t)(args.nchunk - 1) * S.D] = g;
   constexpr int KB = 16;
-  for (int fb = args.nfine; fb > 0; fb -= KB) {
+  for (int kb = args.nchunk - 1; kb > 0; kb -= KB) {
     float A[KB], G[KB];
 #pragma unroll
     for (int q = 0; q < KB; ++q) {
-      const int f = fb - 1 - q;
-      A[q] = f >= 0 ? ap[(int64_t)f * S.D] : 1.0f;
-      G[q] = f >= 0 ? ap[plane + (int64_t)f * S.D] : 0.0f;
+      const int k = kb - q > 0 ? kb - q : 1;
+      A[q] = ap[(int64_t)k * S.D];
+      G[q] = ap[plane + (int64_t)k * S.D];
     }
 #pragma unroll
     for (int q = 0; q < KB; ++q) {
-      const int f = fb - 1 - q;
-      if (f >= 0) {
-        // f is the last sub-chunk of chunk k = f / fpc: g is that chunk's carry
-        const int k = f / fpc;
-        if ((f + 1) % fpc == 0 && k < args.nchunk - 1) cp[(int64_t)k * S.D] = g;
+      const int k = kb - q;
+      if (k > 0) {
         g = fmaf(A[q], g, G[q]);
+        cp[(int64_t)(k - 1) * S.D] = g;
       }
     }
   }
 }
 
+namespace {
+template <typename TIO, bool VEC, bool GL>
+bool launch_bwd_maps(const BwdArgs& a, int grid, hipStream_t st) {
+  const int cl = next_pow2((a.sh.D + Pack<TIO>::V - 1) / Pack<TIO>::V);
+#define LTV_X(CL_)                                                                          \
+  if (cl == CL_) {                                                                          \
+    hipLaunchKernelGGL((scan_bwd_maps_kernel<TIO, VEC, CL_, GL>), dim3(grid), dim3(256), 0, \
+                       st, a);                                                              \
+    return true;                                                                            \
+  }
+  LTV_X(1) LTV_X(2) LTV_X(4) LTV_X(8) LTV_X(16) LTV_X(32) LTV_X(64)
+#undef LTV_X
+  return false;
+}
+template <typename TIO>
+bool launch_bwd_maps_t(const BwdArgs& a, int grid, bool vec, hipStream_t st) {
+  if (a.sh.r % Pack<TIO>::V == 0)
+    return vec ? launch_bwd_maps<TIO, true, true>(a, grid, st)
+               : launch_bwd_maps<TIO, false, true>(a, grid, st);
+  return vec ? launch_bwd_maps<TIO, true, false>(a, grid, st)
+             : launch_bwd_maps<TIO, false, false>(a, grid, st);
+}
+}  // namespace
+
 // The per-chunk maps of the reverse recurrence, then each chunk's carry.
 int scan_launch_bwd_chunk_maps(bool bf16, const BwdArgs& a, bool vec, hipStream_t st) {
   const ScanShape& S = a.sh;
-  const int V = bf16 ? 8 : 4;
-  const int64_t n = (int64_t)S.B * S.H * a.nfine * ((S.D + V - 1) / V);
-  const int blocks = (int)((n + 255) / 256);
-  if (bf16) {
-    if (vec)
-      hipLaunchKernelGGL((scan_bwd_agg_kernel<bf16_t, true>), dim3(blocks), dim3(256), 0, st, a);
-    else
-      hipLaunchKernelGGL((scan_bwd_agg_kernel<bf16_t, false>), dim3(blocks), dim3(256), 0, st, a);
-  } else {
-    if (vec)
-      hipLaunchKernelGGL((scan_bwd_agg_kernel<float, true>), dim3(blocks), dim3(256), 0, st, a);
-    else
-      hipLaunchKernelGGL((scan_bwd_agg_kernel<float, false>), dim3(blocks), dim3(256), 0, st, a);
-  }
+  const int64_t grid = (int64_t)S.B * S.H * (a.nchunk - 1);
+  LTV_REQUIRE(grid < (1ll << 31), LTV_ERR_UNSUPPORTED, "grid too large");
+  const bool ok = bf16 ? launch_bwd_maps_t<bf16_t>(a, (int)grid, vec, st)
+                       : launch_bwd_maps_t<float>(a, (int)grid, vec, st);
+  LTV_REQUIRE(ok, LTV_ERR_UNSUPPORTED, "chunk maps: head_dim %d is not built", S.D);
   LTV_LAUNCH_CHECK();
   const int64_t nc = (int64_t)S.B * S.H * S.D;
-  hipLaunchKernelGGL(scan_bwd_carry_kernel, dim3((int)((nc + 255) / 256)), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(scan_bwd_carry_kernel, dim3((int)((nc + 127) / 128)), dim3(128), 0, st, a);
   LTV_LAUNCH_CHECK();
   return LTV_OK;
 }
@@ -554,17 +565,18 @@ ChainCtl chain_ctl(hipStream_t st) {
   }
   return ChainCtl{h.dev, h.spin_max, h.no_publish};
 }
-// (b, h) sequences from which the backward keeps the tile kernel (which runs
-// unchunked from 256 sequences on).  Measured on MI355X (heads of 128,
-// r = 128, bf16; chained shape L = 4, NW = 4), tile against chained:
-//   B = 32, T = 1024 (576 sequences): 112 against 171 us (L = 4, NW = 2:
-//     242 us) -- 16 chunks per sequence and about two chunk rows resident
-//     make the chain's critical path the time;
-//   B = 16 (288): T = 1024 84 against 89 us, T = 2048 160 against 156 us;
-//   below 256, where the tile kernel needs the chunk-map passes: B = 8 / 4,
-//     T = 1024 (144 / 72) 90 / 72 against 54 / 36 us; B = 8, T = 4096 222
-//     against 157 us; T = 8192: B = 8 / 4 / 2 / 1 (configs[4]'s shape is
-//     B = 8) 400 / 232 / 139 / 108 against 298 / 166 / 120 / 103 us.
+// (b, h) sequences from which the backward keeps the tile kernel, unchunked
+// from there on, although a chain workspace is given.  Measured on MI355X
+// (heads of 128, r = 128, bf16; chained shape L = 4, NW = 4), tile against
+// chained: B = 32, T = 1024 (576 sequences) 112 against 171 us -- 16 chunks per
+// sequence and about two chunk rows resident make the chain's critical path the
+// time; B = 16 (288) T = 1024 84 against 89 us, T = 2048 160 against 156 us;
+// below 256 the tile kernel needs the chunk maps: T = 1024, B = 8 / 4 (16
+// chunks) 53 / 36 against 52 / 34 us.  With more chunks than that the hand-offs
+// (0.75 us each) are the chain's time and the maps win -- callers then pass no
+// chain workspace: T = 16384, B = 1 91 against 194 us (fp32 128 against 369); T =
+// 8192, B = 2 / 8 85 / 266 against 120 / 301 us; T = 4096, B = 4 83 against 90;
+// fp32 B = 8, T = 1024 (32 chunks) 68 against 80 us.
 constexpr int64_t kBwdChainMaxSeqs = 256;
 
 ChainPlan chain_plan(int dtype, int B, int T, int H, int Da, int r) {
@@ -750,24 +762,22 @@ int scan_forward_impl(int dtype, const HostView4& u, const HostView4& lg, const 
   return launch_forward(dtype, a, vec, rm, lg, B, T, NH, NKVH, Da, r, use_sigmoid, st);
 }
 
-// Upper bound on the backward's time chunks per (b, h).  With at least 256
-// (b, h) sequences (one per CU on MI355X) chunking only adds the chunk-map
-// passes (measured: 288 sequences, 1 chunk 132 us, 2-4 chunks 150 us); with
-// fewer (long T, small batch) the sequences are cut into chunks of at least
-// one 64-step tile until about 512 workgroups run (144 sequences at T = 8192:
-// 827 us unchunked, 504 us in 4 chunks).  The
-// launch rounds the chunk length up to whole tiles, which never raises the
-// count above this bound.
+// Upper bound on the backward's time chunks per (b, h).  From 256 (b, h)
+// sequences on (one per CU) the chunk maps' pass over gy costs more than the
+// chunks gain (MI355X, heads of 128, T = 1024, unchunked / 4 chunks: B = 16 75 /
+// 77 us, B = 32 112 / 125 us; T = 2048, B = 24 152 / 200 us).  Below, about 1024
+// workgroups (four of four wavefronts per CU, half of them resident) of at least
+// 128 steps: T = 16384, B = 1 (18 sequences) 8 / 16 / 32 / 64 chunks 160 / 118 /
+// 91 / 91 us; T = 8192, B = 2 114 / 89 / 85 / 96; B = 8, 4 / 8 / 16 / 32 chunks
+// 320 / 266 / 275 / 279 us; T = 1024, B = 4 (128-step chunks against 64-step)
+// 35.8 against 41.6 us.
 int bwd_max_chunks(int B, int H, int T) {
   const int64_t bh = (int64_t)B * H;
   int nc = tuning().bwd_chunks;
-  if (nc == 0) nc = bh >= 256 ? 1 : (int)((512 + bh - 1) / bh);
-  const int cap = (T + 63) / 64;
+  if (nc == 0) nc = bh >= 256 ? 1 : (int)((1024 + bh - 1) / bh);
+  const int cap = (T + 127) / 128;
   return std::max(1, std::min(nc, cap));
 }
-
-// Sub-chunk length of the backward's chunk maps (steps).
-constexpr int kBwdFineSteps = 64;
 
 // The chained backward (scan_bwd_kernel in its CHAIN mode): launch shape,
 // gate mode and chunk count for a head of D channels, or CL = 0 where it is
@@ -879,7 +889,7 @@ BwdWorkspace bwd_workspace_plan(int dtype, int B, int T, int NH, int NKVH, int D
   size_t off = al((size_t)B * H * NP * Da * sizeof(float));
   if (NC > 1) {
     w.agg = off;
-    off += al((size_t)2 * B * H * ((T + kBwdFineSteps - 1) / kBwdFineSteps) * D * sizeof(float));
+    off += al((size_t)2 * B * H * NC * D * sizeof(float));
     w.carry = off;
     off += al((size_t)B * H * NC * D * sizeof(float));
   }
@@ -994,8 +1004,6 @@ int scan_backward_impl(int dtype, const HostView4& u, const HostView4& lg, const
   a.dbias_partial = reinterpret_cast<float*>(wsb + wp.partial);
   a.nchunk = 1;
   a.chunk_steps = T;
-  a.nfine = 1;
-  a.fine_steps = T;
   a.agg = nullptr;
   a.carry = nullptr;
   a.P = P;
@@ -1182,16 +1190,11 @@ int scan_backward_impl(int dtype, const HostView4& u, const HostView4& lg, const
     }
     // time chunks of whole tiles; each chunk enters with its exact gradient
     // carry from the chunk-map kernels
-    // (TW and the sub-chunk length are powers of two: the larger is a multiple
-    // of the smaller)
     const int TW = cfg.NW * (64 / cfg.CL) * cfg.L;
-    const int unit = std::max(TW, kBwdFineSteps);
     const int nc_max = bwd_max_chunks(B, H, T);
     const int per = (T + nc_max - 1) / nc_max;
-    a.chunk_steps = (per + unit - 1) / unit * unit;
+    a.chunk_steps = std::max(2, (per + TW - 1) / TW) * TW;
     a.nchunk = (T + a.chunk_steps - 1) / a.chunk_steps;
-    a.fine_steps = kBwdFineSteps;
-    a.nfine = (T + kBwdFineSteps - 1) / kBwdFineSteps;
     const int64_t grid = (int64_t)B * H * a.nchunk;
     LTV_REQUIRE(grid < (1ll << 31), LTV_ERR_UNSUPPORTED, "grid too large");
     if (a.nchunk > 1) {

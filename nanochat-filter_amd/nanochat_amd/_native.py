@@ -334,6 +334,23 @@ def chain_workspace(device: torch.device, nbytes: int):
     return buf
 
 
+def _chain_pays(nbytes: int, dtype: torch.dtype, B: int, NH: int, NKVH: int, Da: int,
+                r: int) -> bool:
+    """Whether the chained backward is the faster one, given its workspace size
+    (a 256-byte header, one 8-byte word per channel slot of every chunk but a
+    sequence's last).  Every chunk waits for the one after it, about 0.75 us, so
+    with many chunks the tile kernel over chunk maps wins: measured on MI355X in
+    bf16 (chained / maps), 16 chunks 52 / 53 us at 144 sequences and 34 / 36 at
+    72, 64 chunks 90 / 83 at 72, 128 chunks 120 / 85 at 36.  With fewer than 16
+    sequences both are short (47 chunks of 8 sequences 42 / 29 us); the chained
+    form, one launch instead of three, is kept to 48 chunks there."""
+    lanes = 8 if dtype == torch.bfloat16 else 4
+    slots = 1 << (Da * r // lanes - 1).bit_length()
+    nseq = B * (NH + 2 * NKVH)
+    hand_offs = (nbytes - 256) // (8 * nseq * slots * lanes)
+    return hand_offs < (16 if nseq >= 16 else 48)
+
+
 def chain_workspace_for(dtype: torch.dtype, device: torch.device, B: int, T: int, NH: int,
                         NKVH: int, Da: int, r: int, backward: bool = False) -> ChainWorkspace:
     """The chain workspace for this scan shape (pointer None and 0 bytes where
@@ -342,7 +359,7 @@ def chain_workspace_for(dtype: torch.dtype, device: torch.device, B: int, T: int
     size = (lib().ltv_hm_scan_backward_chain_workspace_size if backward
             else lib().ltv_hm_scan_forward_chain_workspace_size)
     nbytes = size(dtype_code(dtype), B, T, NH, NKVH, Da, r)
-    if nbytes == 0:
+    if nbytes == 0 or (backward and not _chain_pays(nbytes, dtype, B, NH, NKVH, Da, r)):
         return _NO_CHAIN
     check_chain_errors()
     buf = chain_workspace(device, nbytes)
