@@ -202,8 +202,9 @@ int ltv_hm_scan_backward(int dtype, const void* combined, const int64_t combined
  *   kernel is used below 256 (b, head) sequences with 16-byte channel
  *   vectors, gate groups of whole lanes (at most 16 per head) or r = 1, and
  *   at least two chunks; elsewhere the size query returns 0 and a workspace
- *   passed is not touched.  With many chunks per sequence (over about 16 of 64
- *   bf16 steps at 128 channels) NULL is the faster choice.
+ *   passed is not touched.  With many chunks per sequence NULL is the faster
+ *   choice: ltv_hm_scan_backward_chain_pays(...) returns 1 where the chained
+ *   kernel is, else 0.
  *   (LTV_SCAN_BWD_CHAIN_CFG="L,NW" forces it, "0" turns it off.)  `workspace` is sized by ltv_hm_scan_backward_workspace_size
  *   as before (it covers either kernel's dbias partials).
  *
@@ -213,6 +214,7 @@ int ltv_hm_scan_backward(int dtype, const void* combined, const int64_t combined
  * ---------------------------------------------------------------------- */
 size_t ltv_hm_scan_backward_chain_workspace_size(int dtype, int B, int T, int NH, int NKVH,
                                                  int Da, int r);
+int ltv_hm_scan_backward_chain_pays(int dtype, int B, int T, int NH, int NKVH, int Da, int r);
 
 int ltv_hm_scan_backward_ws(int dtype, const void* combined, const int64_t combined_strides[3],
                             const void* inits, const int64_t inits_strides[3],

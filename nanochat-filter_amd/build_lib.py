@@ -4,7 +4,8 @@
 
 Compiles each source under ``csrc/`` with hipcc for gfx950 (in parallel) and
 links them into ``nanochat_amd/libnanochat_filter_amd.so``; the roofline
-microbenchmarks of ``csrc/bench/`` go into ``nanochat_amd/libltv_peaks.so``.
+microbenchmarks of ``csrc/bench/`` go into ``nanochat_amd/libltv_peaks.so``, the
+PyTorch host path of ``csrc/torch/`` into ``nanochat_amd/_ltv_torch.so``.
 Always rebuilds.
 """
 
@@ -28,6 +29,35 @@ ARCH = "gfx950"
 # roofline microbenchmarks for bench.py --workload peaks: a library of their own
 PEAKS_SOURCES = ["bench/ltv_peaks.hip"]
 PEAKS_OUT = os.path.join(HERE, "nanochat_amd", "libltv_peaks.so")
+
+
+# host path for PyTorch over the C ABI (no device code)
+TORCH_SOURCES = ["torch/ltv_torch.cpp"]
+TORCH_OUT = os.path.join(HERE, "nanochat_amd", "_ltv_torch.so")
+
+
+def torch_build_command(out: str) -> list[str]:
+    """g++ line of the PyTorch extension: host code only, against the torch that
+    will import it and the library beside it."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    inc = [*include_paths(), os.path.join(rocm_home(), "include"),
+           sysconfig.get_paths()["include"]]
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", "-DTORCH_EXTENSION_NAME=_ltv_torch",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            *[f for i in inc for f in ("-isystem", i)],
+            *[os.path.join(CSRC, s) for s in TORCH_SOURCES], "-o", out,
+            *[f"-L{p}" for p in library_paths()], "-ltorch", "-ltorch_cpu", "-ltorch_python",
+            "-lc10", "-lc10_hip", f"-L{os.path.join(rocm_home(), 'lib')}", "-lamdhip64",
+            f"-L{os.path.dirname(OUT)}", f"-l:{os.path.basename(OUT)}", "-Wl,-rpath,$ORIGIN"]
+
+
+def rocm_home() -> str:
+    return os.path.dirname(os.path.dirname(os.path.realpath(hipcc())))
 
 
 def hipcc() -> str:
@@ -91,6 +121,13 @@ def build(jobs: int | None = None, verbose: bool = True) -> str:
             os.replace(tmp_out, out)
             if verbose:
                 print(f"[build] wrote {out} ({os.path.getsize(out)} bytes)")
+        tmp_out = TORCH_OUT + ".tmp"
+        p = subprocess.run(torch_build_command(tmp_out), capture_output=True, text=True)
+        if p.returncode != 0:
+            raise RuntimeError(f"building the PyTorch extension failed:\n{p.stdout}\n{p.stderr}")
+        os.replace(tmp_out, TORCH_OUT)
+        if verbose:
+            print(f"[build] wrote {TORCH_OUT} ({os.path.getsize(TORCH_OUT)} bytes)")
         return OUT
     finally:
         shutil.rmtree(tmp, ignore_errors=True)

@@ -1430,6 +1430,20 @@ extern "C" size_t ltv_hm_scan_backward_chain_workspace_size(int dtype, int B, in
   return bwd_chain_plan(dtype, B, T, NH + 2 * NKVH, Da, r).bytes;
 }
 
+// Whether the chained backward is the faster one.  Every chunk waits for the one
+// after it, about 0.75 us, so with many chunks the tile kernel over chunk maps
+// wins: measured on MI355X in bf16 (chained / maps), 16 chunks 52 / 53 us at 144
+// sequences and 34 / 36 at 72, 64 chunks 90 / 83 at 72, 128 chunks 120 / 85 at 36.
+// With fewer than 16 sequences both are short (47 chunks of 8 sequences 42 / 29
+// us); the chained form, one launch instead of three, is kept to 48 chunks there.
+extern "C" int ltv_hm_scan_backward_chain_pays(int dtype, int B, int T, int NH, int NKVH, int Da,
+                                               int r) {
+  if (check_shape(dtype, B, T, NH, NKVH, Da, r) != LTV_OK) return 0;
+  const BwdChainPlan p = bwd_chain_plan(dtype, B, T, NH + 2 * NKVH, Da, r);
+  if (p.bytes == 0) return 0;
+  return tuning().bwd_chain_l > 0 || p.nchunk <= (p.nseq >= 16 ? 16 : 48) ? 1 : 0;
+}
+
 extern "C" int ltv_chain_take_error(void) {
   ltv::ChainHost& h = ltv::chain_host();
   std::lock_guard<std::mutex> lk(h.mu);

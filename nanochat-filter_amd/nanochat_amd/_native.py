@@ -110,6 +110,8 @@ SIGNATURES = {
     ),
     "ltv_hm_scan_backward_chain_workspace_size": (
         _c_sz, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int]),
+    "ltv_hm_scan_backward_chain_pays": (
+        _c_int, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int]),
     # the backward with a chain workspace: (chain workspace, bytes) after the workspace
     "ltv_hm_scan_backward_ws": (
         _c_int,
@@ -226,6 +228,26 @@ def lib() -> ctypes.CDLL:
     return _lib if _lib is not None else load()
 
 
+_ext = None
+
+
+def torch_ext():
+    """The native host path of the bf16 filter (``_ltv_torch.so``, built beside the
+    library from ``csrc/torch``): the fused op's autograd function and the decode
+    step without the interpreter.  Raises if it is not built."""
+    global _ext
+    if _ext is None:
+        lib()
+        try:
+            from nanochat_amd import _ltv_torch
+        except ImportError as e:
+            raise RuntimeError(
+                f"_ltv_torch.so is missing or does not load ({e}): build it with "
+                "`python nanochat-filter_amd/build_lib.py` (or __graft_entry__.build())") from e
+        _ext = _ltv_torch
+    return _ext
+
+
 def last_error() -> str:
     return lib().ltv_last_error().decode("utf-8", "replace")
 
@@ -306,10 +328,16 @@ def check_chain_errors() -> None:
     synchronisation).  The chain workspaces are then dropped, so the next
     call starts from a fresh zeroed one."""
     code = lib().ltv_chain_take_error()
-    if code == 0:
-        return
+    if code != 0:
+        raise_chain_error(code)
+
+
+def raise_chain_error(code: int) -> None:
+    """Drop the chain workspaces and raise for the reported error ``code``."""
     torch.cuda.synchronize()
     _CHAIN_WS.clear()
+    if _ext is not None:
+        _ext.drop_chain_workspaces()
     raise RuntimeError(
         f"chained LTV scan failed (code {code}: {CHAIN_ERRORS.get(code, 'unknown')}); the "
         "outputs of chained scan calls since the previous check are invalid, and the chain "
@@ -334,23 +362,6 @@ def chain_workspace(device: torch.device, nbytes: int):
     return buf
 
 
-def _chain_pays(nbytes: int, dtype: torch.dtype, B: int, NH: int, NKVH: int, Da: int,
-                r: int) -> bool:
-    """Whether the chained backward is the faster one, given its workspace size
-    (a 256-byte header, one 8-byte word per channel slot of every chunk but a
-    sequence's last).  Every chunk waits for the one after it, about 0.75 us, so
-    with many chunks the tile kernel over chunk maps wins: measured on MI355X in
-    bf16 (chained / maps), 16 chunks 52 / 53 us at 144 sequences and 34 / 36 at
-    72, 64 chunks 90 / 83 at 72, 128 chunks 120 / 85 at 36.  With fewer than 16
-    sequences both are short (47 chunks of 8 sequences 42 / 29 us); the chained
-    form, one launch instead of three, is kept to 48 chunks there."""
-    lanes = 8 if dtype == torch.bfloat16 else 4
-    slots = 1 << (Da * r // lanes - 1).bit_length()
-    nseq = B * (NH + 2 * NKVH)
-    hand_offs = (nbytes - 256) // (8 * nseq * slots * lanes)
-    return hand_offs < (16 if nseq >= 16 else 48)
-
-
 def chain_workspace_for(dtype: torch.dtype, device: torch.device, B: int, T: int, NH: int,
                         NKVH: int, Da: int, r: int, backward: bool = False) -> ChainWorkspace:
     """The chain workspace for this scan shape (pointer None and 0 bytes where
@@ -359,7 +370,8 @@ def chain_workspace_for(dtype: torch.dtype, device: torch.device, B: int, T: int
     size = (lib().ltv_hm_scan_backward_chain_workspace_size if backward
             else lib().ltv_hm_scan_forward_chain_workspace_size)
     nbytes = size(dtype_code(dtype), B, T, NH, NKVH, Da, r)
-    if nbytes == 0 or (backward and not _chain_pays(nbytes, dtype, B, NH, NKVH, Da, r)):
+    if nbytes == 0 or (backward and not lib().ltv_hm_scan_backward_chain_pays(
+            dtype_code(dtype), B, T, NH, NKVH, Da, r)):
         return _NO_CHAIN
     check_chain_errors()
     buf = chain_workspace(device, nbytes)

@@ -500,10 +500,17 @@ class _QkvFilterEager(torch.autograd.Function):
 def qkv_filter_call(x: torch.Tensor, weight: torch.Tensor, inits: torch.Tensor,
                     logit_bias: torch.Tensor, NH: int, NKVH: int, Da: int, r: int,
                     P: int = UNBOUNDED_P, Q: int = 1, K: int = 1):
-    """``nanochat_amd::qkv_filter`` as the filter modules call it: the library
-    op under ``torch.compile`` (its schema, fake impl and registered autograd),
-    the same implementation through ``_QkvFilterEager`` in eager mode."""
+    """(q, k, v) of ``nanochat_amd::qkv_filter`` as the filter modules call it:
+    the library op under ``torch.compile`` (its schema, fake impl and registered
+    autograd); in eager mode the native autograd function over the same library
+    calls, or ``_QkvFilterEager`` where that one does not take the inputs
+    (tensor subclasses, tracing, transforms, arguments to refuse) or the calls
+    are being timed one by one."""
     if torch.compiler.is_compiling():
         return torch.ops.nanochat_amd.qkv_filter(x, weight, inits, logit_bias, NH, NKVH, Da, r,
-                                                 P, Q, K)
-    return _QkvFilterEager.apply(x, weight, inits, logit_bias, NH, NKVH, Da, r, P, Q, K)
+                                                 P, Q, K)[:3]
+    if N._recorder is None:
+        out = N.torch_ext().qkv_filter(x, weight, inits, logit_bias, NH, NKVH, Da, r, P, Q, K)
+        if out is not None:
+            return out
+    return _QkvFilterEager.apply(x, weight, inits, logit_bias, NH, NKVH, Da, r, P, Q, K)[:3]
