@@ -324,7 +324,11 @@ int launch_gemm_dma(GemmArgs a, const Epi& e, int splits, hipStream_t st) {
   a.splits = splits;
   const int total = a.tiles_i * a.tiles_j * splits;
   if (total == 0) return LTV_OK;
-  int grid = device_cu_count();
+  // as many workgroups as a CU's 160 KB of LDS hold: one of 256 x 256 (or of
+  // 128 x 128 with 8 wavefronts' staging), two of 128 x 128 with 4
+  constexpr int per_cu = (int)(163840 / sizeof(DmaLds<BI, BJ, WGI * WGJ>));
+  static_assert(per_cu >= 1, "the tile's stages exceed the LDS");
+  int grid = per_cu * device_cu_count();
   if (total < grid) grid = total;
   hipLaunchKernelGGL((gemm_dma_kernel<BI, BJ, WGI, WGJ, PL, QL, Epi>), dim3(grid),
                      dim3(WGI * WGJ * 64), 0, st, a, e);
@@ -360,6 +364,7 @@ const GemmTuning& gemm_tuning() {
 }
 
 inline int round_up(int x, int m) { return (x + m - 1) / m * m; }
+inline int tiles128(int i, int j) { return ((i + 127) / 128) * ((j + 127) / 128); }
 
 }  // namespace
 
@@ -675,6 +680,16 @@ extern "C" int ltv_qkv_project_forward(const void* x, const void* wpack, void* v
       a.tiles_i = (Fp + 127) / 128;
       return launch_gemm_dma<128, 256, 2, 4, OP_KC, OP_KC>(a, e, 1, st);
     }
+    // 128 x 128 tiles where two per CU hold them all: 256 x 256 ones then leave
+    // CUs idle, and each CU's serial chain of k-steps sets the time.  us, d12
+    // widths (256 -> 128): M = 512 20.8 -> 12.8, 1024 21.0 -> 13.5, 2048 (304
+    // tiles) 22.3 -> 15.5; M = 5439 of C = 640 (473) 25.7 -> 20.1; past the
+    // line, M = 4096 (608) 24.5 -> 26.6, 16384 70 -> 73.
+    if (gemm_tuning().fwd == 1 && tiles128(Fp, M) <= 2 * device_cu_count()) {
+      a.tiles_i = Fp / 128;
+      a.tiles_j = (M + 127) / 128;
+      return launch_gemm_dma<128, 128, 2, 2, OP_KC, OP_KC>(a, e, 1, st);
+    }
     a.tiles_i = (Fp + 255) / 256;
     return launch_gemm_dma<256, 256, 2, 4, OP_KC, OP_KC>(a, e, 1, st);
   }
@@ -710,6 +725,33 @@ inline int dw_split_rows(int M, int C, int Fp) {
   // per-item overhead and partial sums than they gain in parallelism
   return std::max(1024, round_up((M + S - 1) / S, 64));
 }
+// The dW GEMM outside the fused launch: 128 x 128 tiles, two workgroups per CU,
+// where the plan above leaves half of the CUs without an item -- few tokens, or
+// too few output tiles for 1024-row splits to make up for.  Splits: as many as
+// fit one round, of at least 512 rows.  us with the reduction of the partials
+// (256 -> 128): M = 1024 of d12 (30 items of 256 x 256) 30.8 -> 17.7, 2048 (60)
+// 31.6 -> 25.2, 4096 (120) 34.9 -> 30.5; M = 5439 of C = 640 (108) 32.3 -> 30.7;
+// M = 20000 of C = 256 (60) 31.7 -> 20.4; past the line, M = 8192 of
+// d12 (240) 45.2 -> 48.1.
+struct DwSplit {
+  int rows, S;
+  bool small;
+};
+inline DwSplit dw_split_plan(int M, int C, int Fp) {
+  const GemmTuning& tu = gemm_tuning();
+  DwSplit p;
+  p.rows = dw_split_rows(M, C, Fp);
+  p.S = dw_splits(M, p.rows);
+  const int tiles = ((C + 255) / 256) * (dw_rows(Fp, tu.dw) / 256);
+  p.small = tu.dma && tu.dw == 0 && tu.dw_split == 0 &&
+            (int64_t)tiles * p.S * 2 <= device_cu_count();
+  if (p.small) {
+    const int S = std::max(1, 2 * device_cu_count() / tiles128(C, Fp));
+    p.rows = std::max(512, round_up((M + S - 1) / S, 64));
+    p.S = dw_splits(M, p.rows);
+  }
+  return p;
+}
 // Sum of the S fp32 partials of grad_weight (S slots of Fr x C) into the
 // parameter's interleaved row order.
 int dw_reduce_launch(void* workspace, float* grad_weight, int S, int Fr, int H, int D, int Da,
@@ -737,7 +779,9 @@ int dw_reduce_launch(void* workspace, float* grad_weight, int S, int Fr, int H, 
 extern "C" size_t ltv_qkv_project_backward_workspace_size(int M, int C, int H, int D, int Da) {
   const int Fp = ltv_qkv_packed_width(H, D, Da);
   const GemmTuning& tu = gemm_tuning();
-  return (size_t)dw_splits(M, dw_split_rows(M, C, Fp)) * dw_rows(Fp, tu.dw) * C * sizeof(float);
+  // (the fused launch runs the plan without small tiles)
+  const int S = std::max(dw_splits(M, dw_split_rows(M, C, Fp)), dw_split_plan(M, C, Fp).S);
+  return (size_t)S * dw_rows(Fp, tu.dw) * C * sizeof(float);
 }
 
 namespace {
@@ -796,6 +840,18 @@ int project_backward_input_impl(const void* x, const void* wpack, void* grad_com
         ad.tiles_i = (C + 127) / 128;
         return launch_gemm_dma<128, 256, 2, 4, OP_RC, OP_KC>(ad, e, 1, st);
       }
+      // 128 x 128 tiles where one per CU holds them all, with 8 wavefronts: each
+      // CU runs one serial chain of k-steps, and the second wavefront of a SIMD
+      // hides the first's load issue and LDS latency.  us, d12 widths (256 x 256
+      // -> 128 x 128 with 4 wavefronts -> with 8): M = 512 47.7 -> 37.4 -> 27.6,
+      // 2048 50.0 -> 37.7 -> 30.5, 4096 (192 tiles) 50.0 -> 38.0 -> 30.8;
+      // M = 5439 of C = 640 (215) 32.0 -> 25.6 -> 22.9; past the line, M = 8192
+      // (384) 50.0 -> 48.6 -> 59.4.
+      if (gemm_tuning().dx == 1 && tiles128(C, M) <= device_cu_count()) {
+        ad.tiles_i = (C + 127) / 128;
+        ad.tiles_j = (M + 127) / 128;
+        return launch_gemm_dma<128, 128, 2, 4, OP_RC, OP_KC>(ad, e, 1, st);
+      }
       ad.tiles_i = (C + 255) / 256;
       return launch_gemm_dma<256, 256, 2, 4, OP_RC, OP_KC>(ad, e, 1, st);
     }
@@ -849,16 +905,20 @@ extern "C" int ltv_qkv_project_backward_weight(const void* x, const void* grad_c
   const GemmTuning& tu = gemm_tuning();
   // dW^T[c, f] = sum_m X[m, c] dC[m, f]:  i = c (RC: X[m * C + c]), j = f (RC: dC[m * Fp + f]),
   // the reduction over m split into fp32 partials P_s[f][c]
-  const int split_rows = dw_split_rows(M, C, Fp);
-  const int S = dw_splits(M, split_rows);
+  const DwSplit plan = dw_split_plan(M, C, Fp);
+  const int S = plan.S;
   const int Fr = dw_rows(Fp, tu.dw);
   GemmArgs a;
   a.P = GemmOperand{reinterpret_cast<const bf16_t*>(x), C, C, M};
   a.Q = GemmOperand{reinterpret_cast<const bf16_t*>(grad_combined), Fp, Fp, M};
   a.K = M;
-  a.k_split = split_rows;
+  a.k_split = plan.rows;
   EpiRowF32Split e{reinterpret_cast<float*>(workspace), C, (int64_t)Fr * C, C, Fr};
-  if (tu.dma && dma_usable(a, OP_RC, OP_RC, e, S)) {
+  if (plan.small && dma_usable(a, OP_RC, OP_RC, e, S)) {
+    a.tiles_i = (C + 127) / 128;
+    a.tiles_j = Fp / 128;
+    rc = launch_gemm_dma<128, 128, 2, 2, OP_RC, OP_RC>(a, e, S, st);
+  } else if (tu.dma && dma_usable(a, OP_RC, OP_RC, e, S)) {
     a.tiles_i = (C + 255) / 256;
     a.tiles_j = (Fr + 255) / 256;
     rc = launch_gemm_dma<256, 256, 2, 4, OP_RC, OP_RC>(a, e, S, st);
