@@ -332,7 +332,7 @@ int rows_mode(int dtype, const void* p, const int64_t* s, int T, int D, int r) {
 
 // Launch-shape overrides, read once: LTV_SCAN_FWD_CFG="CL,L,NW" (CL = channel
 // lanes per wavefront, L = steps per lane, NW = wavefronts per workgroup) and
-// LTV_SCAN_BWD_CFG="L,NW" (the backward always spans the whole head).
+// LTV_SCAN_BWD_CFG="L,NW" (the backward then spans the whole head).
 struct ScanTuning {
   int fwd_cl = 0, fwd_l = 0, fwd_nw = 0;
   // LTV_SCAN_CHAIN_CFG="CL,L,NW" (chained forward shape) or "0" (tile kernel only)
@@ -1188,6 +1188,19 @@ int scan_backward_impl(int dtype, const HostView4& u, const HostView4& lg, const
       cfg.L = tu.bwd_l;
       cfg.NW = tu.bwd_nw;
     }
+    // One gate per channel in bf16: the kernel holds 8 gates per lane and step,
+    // so a whole head of 128 channels left one or two wavefronts per SIMD, each
+    // waiting for its tile's loads.  64-channel slabs in workgroups of two
+    // wavefronts give more, independent ones.  Backward at T = 1024 (before ->
+    // here, us):
+    // heads of 128, 288 / 576 / 1152 sequences 139 -> 116, 236 -> 198, 363 ->
+    // 340; heads of 64, 240 / 600 sequences 77 -> 62, 151 -> 124.  32-channel
+    // slabs cut the rows below a 128-byte line (139 / 282 / 547 us).  fp32 (4
+    // gates per lane) gains nothing: 98 -> 103, 203 -> 196, 340 -> 354 us.
+    if (gm == GATE_CHANVEC && dtype == LTV_DTYPE_BF16 && cfg.CL >= 8 && tu.bwd_l == 0) {
+      cfg = ScanCfg{8, 4, 2};
+      a.nslab = (D + 8 * V - 1) / (8 * V);
+    }
     // time chunks of whole tiles; each chunk enters with its exact gradient
     // carry from the chunk-map kernels
     const int TW = cfg.NW * (64 / cfg.CL) * cfg.L;
@@ -1195,7 +1208,7 @@ int scan_backward_impl(int dtype, const HostView4& u, const HostView4& lg, const
     const int per = (T + nc_max - 1) / nc_max;
     a.chunk_steps = std::max(2, (per + TW - 1) / TW) * TW;
     a.nchunk = (T + a.chunk_steps - 1) / a.chunk_steps;
-    const int64_t grid = (int64_t)B * H * a.nchunk;
+    const int64_t grid = (int64_t)B * H * a.nslab * a.nchunk;
     LTV_REQUIRE(grid < (1ll << 31), LTV_ERR_UNSUPPORTED, "grid too large");
     if (a.nchunk > 1) {
       a.agg = reinterpret_cast<float*>(wsb + wp.agg);

@@ -182,6 +182,7 @@ struct BwdArgs {
   uint32_t* ch_err;
   unsigned long long* ch_words;
   ChainCtl ch_ctl;
+  int nslab = 1;  // GATE_CHANVEC tile kernel: workgroups per head, CL V channels each
 };
 
 // How a lane finds the gate of each of its V channels.
@@ -1431,6 +1432,9 @@ scan_bwd_kernel(const BwdArgs args) {
   static_assert(!(CHAIN && LB), "the chained backward runs the full recurrence");
   static_assert(RM == ROWS_NONE || (VEC && GL && !LB), "row modes: one gate per lane, no windows");
   static_assert(!CHAIN || NCH <= NT, "the chain step takes one thread per channel slot");
+  // one gate per channel: nothing crosses a lane's channels, so a head can be
+  // cut into slabs of NCH channels, one workgroup each
+  constexpr bool SLAB = GM == GATE_CHANVEC && !LB && !CHAIN;
   const ScanShape& S = args.sh;
 
   const int lane = threadIdx.x & 63;
@@ -1439,7 +1443,13 @@ scan_bwd_kernel(const BwdArgs args) {
   const int tg = lane % TG;
 
   // one workgroup per (b, head, time chunk): every gate group of the head inside
+  // (per slab of the head with one gate per channel)
   int bh = blockIdx.x / args.nchunk, chunk = blockIdx.x % args.nchunk;
+  int slab = 0;
+  if constexpr (SLAB) {
+    slab = bh % args.nslab;
+    bh /= args.nslab;
+  }
   __shared__ int lds_ticket;
   __shared__ float lds_cin[CHAIN ? NCH : 1];  // the carry entering the chunk
   if constexpr (CHAIN) {
@@ -1467,7 +1477,7 @@ scan_bwd_kernel(const BwdArgs args) {
   const int h = bh % S.H;
   const int b = bh / S.H;
 
-  const int c0 = cl * V;
+  const int c0 = SLAB ? (slab * CL + cl) * V : cl * V;
   const int nvalid = min(V, S.D - c0);
   const bool active = nvalid > 0;
 
@@ -1965,7 +1975,9 @@ scan_bwd_kernel(const BwdArgs args) {
 #pragma unroll
   for (int k = 0; k < (GL ? 1 : V); ++k) lds_red[threadIdx.x][k] = dacc[k];
   __syncthreads();
-  for (int j = threadIdx.x; j < S.Da; j += NT) {
+  const int j_lo = SLAB ? slab * NCH : 0;
+  const int j_hi = SLAB ? min(S.Da, j_lo + NCH) : S.Da;
+  for (int j = j_lo + (int)threadIdx.x; j < j_hi; j += NT) {
     float acc = 0.0f;
     if (GL) {
       // group j's dlogits were emitted by its last channel lane, in every
@@ -1976,7 +1988,7 @@ scan_bwd_kernel(const BwdArgs args) {
     } else {
       // group j is led by channel c = j r: lane cl = c / V, slot c % V, in every
       // time lane (w, tg) of the workgroup
-      const int c = j * S.r;
+      const int c = j * S.r - j_lo;  // (a slab's r is 1)
       const int lcl = c / V, k = c % V;
       for (int ww = 0; ww < NW; ++ww)
         for (int q = 0; q < TG; ++q) acc += lds_red[ww * 64 + lcl * TG + q][k];

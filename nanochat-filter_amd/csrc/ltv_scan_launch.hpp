@@ -138,8 +138,22 @@ bool bwd_dispatch_lb(const BwdArgs& a, int grid, bool vec, int gm, hipStream_t s
   return false;
 }
 
+// The slab shape: one gate per channel, bf16, full recurrence only.
+template <int CL, int L, int NW>
+constexpr bool is_slab_cfg() {
+  return CL == 8 && L == 4 && NW == 2;
+}
+
 template <typename TIO, int CL, int L, int NW>
 bool bwd_dispatch(const BwdArgs& a, int grid, bool vec, int gm, bool lb, int rm, hipStream_t st) {
+  if constexpr (is_slab_cfg<CL, L, NW>()) {
+    if constexpr (sizeof(TIO) == 2) {
+      if (!vec || gm != GATE_CHANVEC || lb || rm != ROWS_NONE) return false;
+      hipLaunchKernelGGL((scan_bwd_kernel<TIO, CL, L, NW, true, GATE_CHANVEC, false>), dim3(grid), dim3(NW * 64), 0, st, a);
+      return true;
+    }
+    return false;
+  }
   if (rm != ROWS_NONE) {
     if constexpr (is_rows_cfg<CL, L, NW>()) {
       const dim3 blk(NW * 64);
@@ -152,8 +166,10 @@ bool bwd_dispatch(const BwdArgs& a, int grid, bool vec, int gm, bool lb, int rm,
     }
     return false;
   }
-  if (!lb) return bwd_dispatch_lb<TIO, CL, L, NW, false>(a, grid, vec, gm, st);
-  if constexpr (is_lb_cfg<CL, L, NW>()) return bwd_dispatch_lb<TIO, CL, L, NW, true>(a, grid, vec, gm, st);
+  if constexpr (!is_slab_cfg<CL, L, NW>()) {
+    if (!lb) return bwd_dispatch_lb<TIO, CL, L, NW, false>(a, grid, vec, gm, st);
+    if constexpr (is_lb_cfg<CL, L, NW>()) return bwd_dispatch_lb<TIO, CL, L, NW, true>(a, grid, vec, gm, st);
+  }
   return false;
 }
 
@@ -191,7 +207,7 @@ bool bwd_chain_dispatch(const BwdArgs& a, int grid, int gm, int rm, hipStream_t 
   X(8, 8, 4) X(8, 2, 4) X(8, 4, 2) X(16, 8, 4) X(4, 8, 4)
 #define LTV_SCAN_BWD_CONFIGS(X)                                                        \
   X(1, 4, 4) X(2, 4, 4) X(4, 4, 4) X(8, 4, 4) X(16, 4, 4) X(32, 4, 4) X(64, 4, 4)      \
-  X(16, 4, 2) X(16, 2, 4)
+  X(16, 4, 2) X(16, 2, 4) X(8, 4, 2)
 
 template <typename TIO>
 int scan_fwd_launch_t(const FwdArgs& a, ScanCfg c, int grid, bool vec, int gm, int rm,

@@ -245,7 +245,8 @@ def backward(ctx, grad_hq, grad_hk, grad_hv):
 
     grad_combined = torch.empty_like(combined)
     grad_inits = torch.empty_like(inits, memory_format=torch.contiguous_format)
-    grad_logit_bias = torch.zeros_like(logit_bias, memory_format=torch.contiguous_format)
+    # every element is written, whatever the sizes: no zeroing launch
+    grad_logit_bias = torch.empty_like(logit_bias, memory_format=torch.contiguous_format)
 
     torch.ops.nanochat_cuda.ltv_fused_concat_head_major_register_cast_blelloch_scan_cuda_backward_kernel(
         combined,

@@ -119,7 +119,8 @@ def allocate_grads(combined, inits, logit_bias, hq, hk, hv, grad_hq, grad_hk, gr
     grad_hv = torch.zeros_like(hv) if grad_hv is None else grad_hv
     grad_combined = torch.empty_like(combined)
     grad_inits = torch.empty_like(inits, memory_format=torch.contiguous_format)
-    grad_logit_bias = torch.zeros_like(logit_bias, memory_format=torch.contiguous_format)
+    # every element is written, whatever the sizes: no zeroing launch
+    grad_logit_bias = torch.empty_like(logit_bias, memory_format=torch.contiguous_format)
     return grad_hq, grad_hk, grad_hv, grad_combined, grad_inits, grad_logit_bias
 
 
