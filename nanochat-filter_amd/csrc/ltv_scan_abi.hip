@@ -124,15 +124,24 @@ int scan_launch_bwd_chain(bool bf16, const BwdArgs& a, ScanCfg cfg, int grid, in
               : scan_bwd_chain_launch_f32(a, cfg, grid, gm, rm, st);
 }
 
-int scan_launch_lb_fold(bool bf16, const BwdArgs& a, hipStream_t st) {
+// vec: D a multiple of 16-byte vectors and du addressable in them
+int scan_launch_lb_fold(bool bf16, const BwdArgs& a, bool vec, hipStream_t st) {
   const ScanShape& S = a.sh;
-  const int64_t n = (int64_t)S.B * S.H * a.nchunk * a.kw * (S.D + S.Da);
-  const int64_t blocks = (n + 255) / 256;
+  const int V = bf16 ? Pack<bf16_t>::V : Pack<float>::V;
+  const int64_t rows = (int64_t)S.B * S.H * a.nchunk * a.kw;
+  const int64_t nvec = rows * (S.D / V + S.Da);
+  vec = vec && nvec < (1ll << 31);  // 32-bit indexes
+  const int64_t blocks = ((vec ? nvec : rows * (S.D + S.Da)) + 255) / 256;
   LTV_REQUIRE(blocks < (1ll << 31), LTV_ERR_UNSUPPORTED, "look-back warm-up too large");
-  if (bf16)
-    hipLaunchKernelGGL(scan_lb_fold_kernel<bf16_t>, dim3((int)blocks), dim3(256), 0, st, a);
+  const dim3 grid((unsigned)blocks), blk(256);
+  if (bf16 && vec)
+    hipLaunchKernelGGL((scan_lb_fold_kernel<bf16_t, true>), grid, blk, 0, st, a);
+  else if (bf16)
+    hipLaunchKernelGGL((scan_lb_fold_kernel<bf16_t, false>), grid, blk, 0, st, a);
+  else if (vec)
+    hipLaunchKernelGGL((scan_lb_fold_kernel<float, true>), grid, blk, 0, st, a);
   else
-    hipLaunchKernelGGL(scan_lb_fold_kernel<float>, dim3((int)blocks), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((scan_lb_fold_kernel<float, false>), grid, blk, 0, st, a);
   LTV_LAUNCH_CHECK();
   return LTV_OK;
 }
@@ -1145,7 +1154,7 @@ int scan_backward_impl(int dtype, const HostView4& u, const HostView4& lg, const
     rc = scan_launch_bwd(bf16, a, cfg, (int)grid, vec, gm, true, ROWS_NONE, st);
     if (rc) return rc;
     if (a.kw > 0) {
-      rc = scan_launch_lb_fold(bf16, a, st);
+      rc = scan_launch_lb_fold(bf16, a, vec, st);
       if (rc) return rc;
     }
     rc = scan_launch_lb_dinit(bf16, a, st);

@@ -2128,47 +2128,80 @@ __global__ void __launch_bounds__(256) scan_bwd_maps_kernel(const BwdArgs args) 
 // ... while lo_c <= t, where c0(t) is the first window starting after t.  Its
 // gradient is the owning window's (already in du / dlg, written by the LB tile
 // kernel) plus those windows' fp32 contributions, added in window order and
-// rounded once.  One thread per (b h, window, warm-up row, channel of the
-// D + Da value and logit slots); the thread whose window is c0(t) does the sum,
-// so each step is written by exactly one thread.
+// rounded once.  One thread per (b h, window, warm-up row, slot); the thread
+// whose window is c0(t) does the sum, so each step is written by exactly one
+// thread.  A row's slots: its value channels, 16 bytes of du (VEC) or one each,
+// then its Da logit slots.
+// Bound by its threads' index arithmetic (64-bit divisions) and one-element
+// accesses while it took a channel per thread: 17.5 us for 19 MB (B = 8, T =
+// 1024, 18 heads of 128, 9 windows with 16 warm-up rows); with 32-bit indexes
+// and a vector per thread 6.5 us.
 // ---------------------------------------------------------------------------
-template <typename TIO>
+template <typename TIO, bool VEC>
 __global__ void __launch_bounds__(256) scan_lb_fold_kernel(const BwdArgs args) {
+  using Index = std::conditional_t<VEC, uint32_t, uint64_t>;
+  constexpr int W = VEC ? Pack<TIO>::V : 1;
   const ScanShape& S = args.sh;
   const int nw = args.nchunk;
-  const int nch = S.D + S.Da;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)S.B * S.H * nw * args.kw * nch) return;
-  const int ch = (int)(idx % nch);
-  int64_t rest = idx / nch;
-  const int row = (int)(rest % args.kw);
-  rest /= args.kw;
-  const int win = (int)(rest % nw);
-  const int64_t bh = rest / nw;
+  const int nvs = S.D / W;  // value slots
+  const Index nslot = (Index)(nvs + S.Da);
+  const Index idx = (Index)blockIdx.x * 256u + threadIdx.x;
+  if (idx >= (Index)S.B * S.H * nw * args.kw * nslot) return;
+  const int slot = (int)(idx % nslot);
+  Index rest = idx / nslot;
+  const int row = (int)(rest % (Index)args.kw);
+  rest /= (Index)args.kw;
+  const int win = (int)(rest % (Index)nw);
+  const int64_t bh = (int64_t)(rest / (Index)nw);
   if (win == 0) return;  // the first window has no warm-up
   const Window wd = look_back_window(win, S.T, args.P, args.Q, args.K);
   const int t = wd.lo + row;
   if (t >= wd.st) return;
   const int cfirst = t < args.P ? 1 : (t - args.P) / args.Q + 2;  // first window with st > t
   if (win != cfirst) return;
-  const int h = (int)(bh % S.H), b = (int)(bh / S.H);
-  TIO* gp;
-  if (ch < S.D) {
-    gp = reinterpret_cast<TIO*>(const_cast<void*>(args.du.p)) + (int64_t)b * args.du.s[0] +
-         (int64_t)h * args.du.s[1] + (int64_t)t * args.du.s[2] + (int64_t)ch * args.du.s[3];
+  const int h = (int)bh % S.H, b = (int)bh / S.H;
+  // f(r) for the rows r of the windows whose warm-up holds t, in window order
+  auto rows = [&](auto&& f) {
+    for (int c = win; c < nw; ++c) {
+      const Window wc = look_back_window(c, S.T, args.P, args.Q, args.K);
+      if (wc.lo > t) break;
+      f((bh * nw + c) * args.kw + (t - wc.lo));
+    }
+  };
+  if (slot >= nvs) {
+    const int j = slot - nvs;
+    TIO* gp = reinterpret_cast<TIO*>(const_cast<void*>(args.dlg.p)) + (int64_t)b * args.dlg.s[0] +
+              (int64_t)h * args.dlg.s[1] + (int64_t)t * args.dlg.s[2] + (int64_t)j * args.dlg.s[3];
+    float acc = Pack<TIO>::load1(gp);
+    rows([&](int64_t r) { acc += args.wdl[r * S.Da + j]; });
+    Pack<TIO>::store1(gp, acc);
+    return;
+  }
+  TIO* gp = reinterpret_cast<TIO*>(const_cast<void*>(args.du.p)) + (int64_t)b * args.du.s[0] +
+            (int64_t)h * args.du.s[1] + (int64_t)t * args.du.s[2] +
+            (int64_t)(slot * W) * args.du.s[3];
+  if constexpr (VEC) {
+    const uint4 q = *reinterpret_cast<const uint4*>(gp);
+    float acc[W];
+#pragma unroll
+    for (int v = 0; v < W; ++v) acc[v] = Pack<TIO>::get(q, v);
+    rows([&](int64_t r) {
+      const float4* wp = reinterpret_cast<const float4*>(args.wdu + r * S.D + slot * W);
+#pragma unroll
+      for (int k = 0; k < W / 4; ++k) {
+        const float4 x = wp[k];
+        acc[4 * k] += x.x;
+        acc[4 * k + 1] += x.y;
+        acc[4 * k + 2] += x.z;
+        acc[4 * k + 3] += x.w;
+      }
+    });
+    *reinterpret_cast<uint4*>(gp) = Pack<TIO>::pack(acc);
   } else {
-    gp = reinterpret_cast<TIO*>(const_cast<void*>(args.dlg.p)) + (int64_t)b * args.dlg.s[0] +
-         (int64_t)h * args.dlg.s[1] + (int64_t)t * args.dlg.s[2] +
-         (int64_t)(ch - S.D) * args.dlg.s[3];
+    float acc = Pack<TIO>::load1(gp);
+    rows([&](int64_t r) { acc += args.wdu[r * S.D + slot]; });
+    Pack<TIO>::store1(gp, acc);
   }
-  float acc = Pack<TIO>::load1(gp);
-  for (int c = win; c < nw; ++c) {
-    const Window wc = look_back_window(c, S.T, args.P, args.Q, args.K);
-    if (wc.lo > t) break;
-    const int64_t r = (bh * nw + c) * args.kw + (t - wc.lo);
-    acc += ch < S.D ? args.wdu[r * S.D + ch] : args.wdl[r * S.Da + (ch - S.D)];
-  }
-  Pack<TIO>::store1(gp, acc);
 }
 
 // grad_inits[b, h, d] = sum over the non-empty windows of their fp32
@@ -2410,7 +2443,7 @@ int scan_launch_bwd(bool bf16, const BwdArgs& a, ScanCfg cfg, int grid, bool vec
 int scan_launch_bwd_chain(bool bf16, const BwdArgs& a, ScanCfg cfg, int grid, int gm, int rm,
                           hipStream_t st);
 // Look-back backward: warm-up contributions into du / dlg, then grad_inits.
-int scan_launch_lb_fold(bool bf16, const BwdArgs& a, hipStream_t st);
+int scan_launch_lb_fold(bool bf16, const BwdArgs& a, bool vec, hipStream_t st);
 int scan_launch_lb_dinit(bool bf16, const BwdArgs& a, hipStream_t st);
 // Short-window look-back kernels (ltv_scan_lb.hip): one lane per (b, h,
 // window, channel vector).  The backward also needs kw_max >= K - 1 (8 or 16).
