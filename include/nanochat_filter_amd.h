@@ -392,8 +392,9 @@ int ltv_hm_look_back_scan_backward_split_ws(
  * x (B, T, K), weight (F, K), out (B, F, T): all contiguous, all `dtype`.
  * bf16 with T a multiple of 256 and K of 8 (16-byte aligned buffers) runs on
  * bf16 MFMA (fp32 accumulation) and writes the (B, F, T) layout directly; fp32
- * and the other bf16 shapes run on fp32 MFMA (v_mfma_f32_32x32x2_f32, fp32
- * accumulation, any sizes and alignment).  x and weight may be NULL when
+ * and the other bf16 shapes run on a strided GEMM (each fp32 operand as three
+ * bf16 pieces, six bf16 MFMA terms per product, fp32 accumulation; any sizes
+ * and alignment).  x and weight may be NULL when
  * K = 0 (out is then zeros).
  * Replaces fused_linear_transpose (cpp_ewma/src/fused_linear_transpose_forward.cu:23-58,
  * called from nanochat/ops/fused_linear_transpose.py:20-40).
@@ -406,7 +407,7 @@ int ltv_linear_transpose_forward(int dtype, const void* x, const void* weight, v
  * `dtype`, fp32 accumulation).
  * grad_out is (B, F, T) contiguous, or its (B, T, F)-contiguous transpose
  * when grad_out_is_btf != 0 (the two layouts the reference accepts,
- * nanochat/ops/fused_linear_transpose.py:76-84).  Runs on fp32 MFMA, the
+ * nanochat/ops/fused_linear_transpose.py:76-84).  Runs on the strided GEMM, the
  * weight gradient in one pass per output tile.  Pointers of tensors with no
  * elements may be NULL.
  * Replaces fused_linear_transpose_backward

@@ -6,7 +6,7 @@ inputs, a zero-initialised (B, F, T) output from the functional op, and a
 backward that accepts grad_out either contiguous or as the transposed view of a
 (B, T, F)-contiguous tensor.  The work runs in the gfx950 library
 (``ltv_linear_transpose_forward`` / ``ltv_linear_transpose_backward_ws``): bf16
-MFMA kernels where the layout allows, else the strided fp32-MFMA GEMM.
+MFMA kernels where the layout allows, else the strided split GEMM.
 """
 
 import torch
