@@ -157,6 +157,67 @@ __device__ __forceinline__ float4 ld_stream4(const float4* p) {
   return make_float4(q[0], q[1], q[2], q[3]);
 }
 
+// p[0] + p[stride] + ... (S terms, in that order), 8 loads at a time
+__device__ __forceinline__ float4 sum_splits4(const float4* p, int S, int64_t split_stride4) {
+      float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      int s = 0;
+      for (; s + 8 <= S; s += 8) {
+        float4 v[8];
+  #pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = ld_stream4(&p[(int64_t)(s + j) * split_stride4]);
+  #pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          acc.x += v[j].x;
+          acc.y += v[j].y;
+          acc.z += v[j].z;
+          acc.w += v[j].w;
+        }
+      }
+      for (; s < S; ++s) {
+        const float4 v = ld_stream4(&p[(int64_t)s * split_stride4]);
+        acc.x += v.x;
+        acc.y += v.y;
+        acc.z += v.z;
+        acc.w += v.w;
+      }
+  return acc;
+}
+
+// reduce_splits_kernel, 4 elements per thread (n and the split stride multiples
+// of 4, 16-byte aligned buffers): the same additions in the same order.  Bound
+// by the partials' bytes.  2322 x 768 in bf16 over 8 partials 13.4 -> 9.8 us,
+// against one element per thread and load.
+template <typename TO>
+__global__ void __launch_bounds__(256)
+reduce_splits4_kernel(const float4* __restrict__ part, TO* __restrict__ out, int S,
+                      int64_t split_stride4, int64_t n4) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n4;
+       i += (int64_t)gridDim.x * 256) {
+    const float4 v = sum_splits4(part + i, S, split_stride4);
+    if constexpr (sizeof(TO) == 4)
+      reinterpret_cast<float4*>(out)[i] = v;
+    else
+      reinterpret_cast<uint2*>(out)[i] = make_uint2(cvt_pk_bf16(v.x, v.y), cvt_pk_bf16(v.z, v.w));
+  }
+}
+
+template <typename TO>
+int launch_reduce_splits(const void* part, void* out, int S, int64_t split_stride, int64_t n,
+                         hipStream_t st) {
+  const bool vec = n % 4 == 0 && split_stride % 4 == 0 && aligned16(part) && aligned16(out);
+  const int blocks = (int)std::min<int64_t>(((vec ? n / 4 : n) + 255) / 256, 8192);
+  if (vec)
+    hipLaunchKernelGGL(reduce_splits4_kernel<TO>, dim3(blocks), dim3(256), 0, st,
+                       reinterpret_cast<const float4*>(part), reinterpret_cast<TO*>(out), S,
+                       split_stride / 4, n / 4);
+  else
+    hipLaunchKernelGGL(reduce_splits_kernel<TO>, dim3(blocks), dim3(256), 0, st,
+                       reinterpret_cast<const float*>(part), reinterpret_cast<TO*>(out), S,
+                       split_stride, n);
+  LTV_LAUNCH_CHECK();
+  return LTV_OK;
+}
+
 __global__ void __launch_bounds__(256)
 dw_reduce4_kernel(const float4* __restrict__ part, float4* __restrict__ gw, int S,
                   int64_t split_stride4, int H, int D, int Da, int C4) {
@@ -166,29 +227,7 @@ dw_reduce4_kernel(const float4* __restrict__ part, float4* __restrict__ gw, int 
     const int f = i / C4, c = i - f * C4;
     const int h = f / DE, e = f - h * DE;
     const int fpk = e < D ? h * D + e : H * D + h * Da + (e - D);
-    const float4* p = part + (int64_t)fpk * C4 + c;
-    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    int s = 0;
-    for (; s + 8 <= S; s += 8) {
-      float4 v[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = ld_stream4(&p[(int64_t)(s + j) * split_stride4]);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        acc.x += v[j].x;
-        acc.y += v[j].y;
-        acc.z += v[j].z;
-        acc.w += v[j].w;
-      }
-    }
-    for (; s < S; ++s) {
-      const float4 v = ld_stream4(&p[(int64_t)s * split_stride4]);
-      acc.x += v.x;
-      acc.y += v.y;
-      acc.z += v.z;
-      acc.w += v.w;
-    }
-    gw[i] = acc;
+    gw[i] = sum_splits4(part + (int64_t)fpk * C4 + c, S, split_stride4);
   }
 }
 
@@ -504,17 +543,9 @@ int lt_backward_split(int dtype, const void* x, const void* weight, const void* 
   rc = launch_w(LTV_DTYPE_F32, S);
   if (rc) return rc;
   const int64_t n = (int64_t)F * K;
-  const int blocks = (int)std::min<int64_t>((n + 255) / 256, 8192);
-  if (dtype == LTV_DTYPE_F32)
-    hipLaunchKernelGGL(reduce_splits_kernel<float>, dim3(blocks), dim3(256), 0, st,
-                       reinterpret_cast<const float*>(workspace),
-                       reinterpret_cast<float*>(grad_weight), S, n, n);
-  else
-    hipLaunchKernelGGL(reduce_splits_kernel<bf16_t>, dim3(blocks), dim3(256), 0, st,
-                       reinterpret_cast<const float*>(workspace),
-                       reinterpret_cast<bf16_t*>(grad_weight), S, n, n);
-  LTV_LAUNCH_CHECK();
-  return LTV_OK;
+  return dtype == LTV_DTYPE_F32
+             ? launch_reduce_splits<float>(workspace, grad_weight, S, n, n, st)
+             : launch_reduce_splits<bf16_t>(workspace, grad_weight, S, n, n, st);
 }
 }  // namespace
 
@@ -597,12 +628,9 @@ extern "C" int ltv_linear_transpose_backward_ws(int dtype, const void* x, const 
     a.tiles_j = sp.Fr / 256;
     int rc = launch_gemm_dma<256, 256, 2, 4, OP_RC, OP_KC>(a, e, sp.S, st);
     if (rc) return rc;
-    const int64_t n = (int64_t)F * K;
-    const int blocks = (int)std::min<int64_t>((n + 255) / 256, 8192);
-    hipLaunchKernelGGL(reduce_splits_kernel<bf16_t>, dim3(blocks), dim3(256), 0, st,
-                       reinterpret_cast<const float*>(workspace),
-                       reinterpret_cast<bf16_t*>(grad_weight), sp.S, (int64_t)sp.Fr * K, n);
-    LTV_LAUNCH_CHECK();
+    rc = launch_reduce_splits<bf16_t>(workspace, grad_weight, sp.S, (int64_t)sp.Fr * K,
+                                      (int64_t)F * K, st);
+    if (rc) return rc;
   }
   return LTV_OK;
 }

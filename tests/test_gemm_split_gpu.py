@@ -72,3 +72,12 @@ def test_f32_non_finite(T):
     mag = torch.matmul(w.double().abs().unsqueeze(0), x.double().abs().transpose(1, 2))
     assert bool(((out.double() - want).abs()[fin] <= (K + 4) * 2.0 ** -24 * mag[fin]).all())
     assert float(out[3, 17, 1]) > 1e30
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "bf16"])
+@pytest.mark.parametrize("T,K,F", [(1024, 64, 98), (1024, 64, 97), (1024, 9, 33), (4096, 32, 257)])
+def test_split_reduction_widths(dtype, T, K, F):
+    """grad_weight's partials summed 4 elements per thread and (F K not a
+    multiple of 4) one by one; one to many splits."""
+    for B in (1, 3, 24):
+        _run(B, T, K, F, dtype, False, seed=F)
