@@ -47,13 +47,51 @@ void* current_stream(const Tensor& t) {
 // and stream, shared with the Python calls on that stream), remembered here so
 // that the interpreter is only entered for a stream's first buffer or a larger
 // one.  _native drops them here too when it drops its own after an error.
+//
+// The buffers are Python's tensors: releasing one may take the interpreter lock,
+// which a thread that wants `mu` may hold.  So none is released under `mu`, and
+// `mu` is never waited for with the interpreter lock held.
 // ---------------------------------------------------------------------------
-std::mutex g_chain_mu;
-std::map<std::pair<int, void*>, Tensor> g_chain;
+using ChainKey = std::pair<int, void*>;  // device, stream
+struct ChainCache {
+  std::mutex mu;
+  std::map<ChainKey, Tensor> bufs;
+  uint64_t drops = 0;  // how often all of them were dropped
+};
+ChainCache& chain_cache() {
+  static ChainCache* c = new ChainCache;  // (outlives the interpreter and the device)
+  return *c;
+}
 
+// The remembered buffer if it is large enough, and the count of drops so far.
+std::pair<Tensor, uint64_t> find_chain_workspace(const ChainKey& key, size_t bytes) {
+  ChainCache& c = chain_cache();
+  std::lock_guard<std::mutex> lk(c.mu);
+  auto it = c.bufs.find(key);
+  const bool hit = it != c.bufs.end() && (size_t)it->second.numel() >= bytes;
+  return {hit ? it->second : Tensor(), c.drops};
+}
+
+// Remembers buf, unless the buffers were dropped since `drops` was read (buf may
+// then be one of the dropped).  The one it replaces is released by the caller.
+Tensor keep_chain_workspace(const ChainKey& key, Tensor buf, uint64_t drops) {
+  ChainCache& c = chain_cache();
+  std::lock_guard<std::mutex> lk(c.mu);
+  if (c.drops == drops) std::swap(c.bufs[key], buf);
+  return buf;
+}
+
+// (called with the interpreter lock)
 void drop_chain_workspaces() {
-  std::lock_guard<std::mutex> lk(g_chain_mu);
-  g_chain.clear();
+  ChainCache& c = chain_cache();
+  std::map<ChainKey, Tensor> old;
+  pybind11::gil_scoped_release nogil;
+  {
+    std::lock_guard<std::mutex> lk(c.mu);
+    old.swap(c.bufs);
+    ++c.drops;
+  }
+  old.clear();
 }
 
 // An earlier chained launch failed: let _native reset the workspaces and raise.
@@ -70,11 +108,12 @@ Tensor chain_workspace(const Tensor& like, void* stream, size_t bytes) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   const bool capturing = hipStreamIsCapturing((hipStream_t)stream, &cs) != hipSuccess ||
                          cs != hipStreamCaptureStatusNone;
-  const std::pair<int, void*> key(like.device().index(), stream);
+  const ChainKey key(like.device().index(), stream);
+  uint64_t drops = 0;
   if (!capturing) {
-    std::lock_guard<std::mutex> lk(g_chain_mu);
-    auto it = g_chain.find(key);
-    if (it != g_chain.end() && (size_t)it->second.numel() >= bytes) return it->second;
+    auto [kept, n] = find_chain_workspace(key, bytes);
+    if (kept.defined()) return kept;
+    drops = n;
   }
   Tensor buf;
   {
@@ -83,10 +122,7 @@ Tensor chain_workspace(const Tensor& like, void* stream, size_t bytes) {
               .attr("chain_workspace")(pybind11::cast(like).attr("device"), bytes)
               .cast<Tensor>();
   }
-  if (!capturing) {
-    std::lock_guard<std::mutex> lk(g_chain_mu);
-    g_chain[key] = buf;
-  }
+  if (!capturing) keep_chain_workspace(key, buf, drops);
   return buf;
 }
 
@@ -335,4 +371,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("qkv_filter", &qkv_filter);
   m.def("decode_rows", &decode_rows);
   m.def("drop_chain_workspaces", &drop_chain_workspaces);
+  // the workspace cache by itself, any tensors (its locking is tested without a device)
+  m.def("_find_chain_workspace", [](int device, int64_t stream, size_t bytes) {
+    return find_chain_workspace({device, reinterpret_cast<void*>(stream)}, bytes);
+  }, pybind11::call_guard<pybind11::gil_scoped_release>());
+  m.def("_keep_chain_workspace", [](int device, int64_t stream, Tensor buf, uint64_t drops) {
+    keep_chain_workspace({device, reinterpret_cast<void*>(stream)}, std::move(buf), drops);
+  }, pybind11::call_guard<pybind11::gil_scoped_release>());
 }
