@@ -8,14 +8,15 @@
 //   A(m, ko, ki) at A + m sam + ko sako + ki saki (+ z sab for batch z), B alike
 //
 // fp32 operands are split exactly into three bf16 pieces, x = x1 + x2 + x3 (each
-// the rest rounded to nearest: 8 + 8 + 8 bits of the significand), and a
+// the rest rounded to nearest: 8 + 8 + 8 bits of the significand; scaled, so that
+// subnormal pieces lose no bits either: kSplitScale), and a
 // product is six MFMA terms, smallest first: x3 y1, x1 y3, x2 y2, x2 y1, x1 y2,
 // x1 y1.  The three left out are below 2^-26 of the product -- under the rounding
 // of one fp32 addition (2^-24 of the sum) that every partial sum takes anyway.
 // A bf16 MFMA term is 16 times as fast as the fp32 MFMA (2.5 against 0.157
 // PFLOP/s nominal), six of them 2.7 times.  Non-finite results send the
 // wavefront's part of the tile through the fp32 MFMA instead (an infinity has
-// no such split, nor has a value that rounds past the largest bf16), so
+// no such split, nor has a value that the scale takes past the largest bf16), so
 // infinities and NaNs come out as fp32 arithmetic gives them.
 // bf16 operands are one piece: the products are exact, as they always were.
 //
@@ -65,6 +66,14 @@ enum SplitLayout { kSplitKC = 0, kSplitRC = 1 };
 
 constexpr int kSplitThreads = 256;  // 4 wavefronts, 2 x 2
 constexpr int kSplitWgPerCu = 3;
+
+// fp32 operands are split at 2^24 times their value: the last bit of the
+// smallest subnormal then lies at 2^-125, so every piece of every operand is a
+// normal bf16 number or zero and the split is exact.  Sums are scaled back once,
+// when they are stored.  (Operands from 2^104 and sums from 2^80 on overflow so
+// and take the non-finite path.)
+constexpr float kSplitScale = 16777216.0f;
+constexpr float kSplitUnscale = 1.0f / (kSplitScale * kSplitScale);
 
 // Pieces per element, and the k-step of a tile of R = 128 or 64 rows.
 template <typename TI>
@@ -227,7 +236,7 @@ struct SplitStager {
         if (cut) shift_down<8, 1>(o.w[c], early);
         float x[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = __uint_as_float(o.w[c][e]);
+        for (int e = 0; e < 8; ++e) x[e] = __uint_as_float(o.w[c][e]) * kSplitScale;
         static_for<NP>([&](auto pc) {
           constexpr int p = decltype(pc)::value;
           uint32_t q[4];
@@ -501,6 +510,13 @@ gemm_split_kernel(const SplitArgs g) {
             split_block_f32(oa, ob, mb, nb, ko, wpb * BK, g.kin, lane, c);
           acc[a][b] = c;
         }
+    } else {
+#pragma unroll
+      for (int a = 0; a < WB; ++a)
+#pragma unroll
+        for (int b = 0; b < WB; ++b)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[a][b][v] *= kSplitUnscale;
     }
   }
 

@@ -81,3 +81,49 @@ def test_split_reduction_widths(dtype, T, K, F):
     multiple of 4) one by one; one to many splits."""
     for B in (1, 3, 24):
         _run(B, T, K, F, dtype, False, seed=F)
+
+
+def _scaled(t, e):
+    """t 2^e in fp32, subnormals included."""
+    return (t.double() * 2.0 ** e).float()
+
+
+@pytest.mark.parametrize("other", [0, 60, 90])
+@pytest.mark.parametrize("e", [-100, -109, -113, -118, -124, -130, -140])
+def test_f32_small_operands(e, other):
+    """Operands down to the smallest subnormals keep every bit, against ordinary
+    and against large ones.  Bound: one fp32 rounding per term of the products
+    (as for any magnitude) and one of 2^-150 per term where results are subnormal."""
+    B, T, K, F = 2, 150, 40, 70
+    x, w, go = _operands(B, T, K, F, torch.float32, 11)
+    x, w = _scaled(x, e), _scaled(w, other)
+    ops = _ops().nanochat_cuda
+    # the small operand on either side: x w^T, and w x^T
+    for a, b in ((x, w), (w.expand(2, F, K).contiguous(), x[0])):
+        out = ops.fused_linear_transpose_cuda_op(a, b)
+        want = torch.matmul(b.double().unsqueeze(0), a.double().transpose(1, 2).contiguous())
+        mag = torch.matmul(b.double().abs().unsqueeze(0),
+                           a.double().abs().transpose(1, 2).contiguous())
+        err = (out.double() - want).abs()
+        assert bool((err <= (K + 1) * (2.0 ** -24 * mag + 2.0 ** -150)).all()), float((err / mag).max())
+    # gradients of the same
+    gx, gw = torch.empty_like(x), torch.empty_like(w)
+    go = _scaled(go, other)
+    ops.fused_linear_transpose_backward_kernel(x, w, go, gx, gw)
+    gd = go.double().permute(1, 0, 2).reshape(F, B * T)
+    xd = x.double().reshape(B * T, K)
+    err, mag = (gw.double() - gd @ xd).abs(), gd.abs() @ xd.abs()
+    assert bool((err <= (B * T + 1) * (2.0 ** -24 * mag + 2.0 ** -150)).all()), float((err / mag).max())
+
+
+def test_f32_values_that_the_scale_overflows():
+    """Finite operands and results past the scaled range come out as usual."""
+    B, T, K, F = 2, 40, 24, 70
+    x, w, _ = _operands(B, T, K, F, torch.float32, 12)
+    for ex, ew in ((105, 0), (60, 40), (0, 81), (103, -90)):
+        a, b = _scaled(x, ex), _scaled(w, ew)
+        out = _ops().nanochat_cuda.fused_linear_transpose_cuda_op(a, b)
+        want = torch.matmul(b.double().unsqueeze(0), a.double().transpose(1, 2).contiguous())
+        mag = torch.matmul(b.double().abs().unsqueeze(0),
+                           a.double().abs().transpose(1, 2).contiguous())
+        assert bool(((out.double() - want).abs() <= (K + 1) * 2.0 ** -24 * mag).all())
