@@ -11,25 +11,33 @@
 // the rest rounded to nearest: 8 + 8 + 8 bits of the significand; scaled, so that
 // subnormal pieces lose no bits either: kSplitScale), and a
 // product is six MFMA terms, smallest first: x3 y1, x1 y3, x2 y2, x2 y1, x1 y2,
-// x1 y1.  The three left out are below 2^-26 of the product -- under the rounding
-// of one fp32 addition (2^-24 of the sum) that every partial sum takes anyway.
+// x1 y1.  The three left out come to at most 2^-24 of a product (x2 y3 and x3 y2
+// 2^-25 each), 2^-27.5 in the mean.  The bf16 MFMA does not round its sums
+// correctly: of two addends the smaller is cut below the last bit of the larger.
+// So the terms of a step of 16 indices are summed by themselves, from zero, and a
+// step's sum enters the accumulator with one fp32 rounding: K / 16 of them, where
+// the fp32 MFMA takes K / 2.  Worst case (K / 16 + 8) 2^-24 of the sum of the
+// products' magnitudes; reductions of up to 16 indices, where that is more than
+// the fp32 arithmetic's K 2^-24, run on the fp32 MFMA (split_blocks_f32).
 // A bf16 MFMA term is 16 times as fast as the fp32 MFMA (2.5 against 0.157
 // PFLOP/s nominal), six of them 2.7 times.  Non-finite results send the
-// wavefront's part of the tile through the fp32 MFMA instead (an infinity has
+// wavefront's part of the tile through the fp32 MFMA too (an infinity has
 // no such split, nor has a value that the scale takes past the largest bf16), so
 // infinities and NaNs come out as fp32 arithmetic gives them.
 // bf16 operands are one piece: the products are exact, as they always were.
 //
 // Measured on MI355X against the fp32-MFMA kernel before it (128 x 128 tiles,
 // quads, one element per load off a 16-byte boundary), 2-norm errors against
-// float64:
-//   fp32 B = 32, T = 1024, K = 768, F = 2322: forward 1070 -> 712 us (164
-//     TFLOP/s), both gradients 2030 -> 1256 us (186); errors 5.0e-7 -> 4.2e-7
-//     (forward), 8.6e-7 -> 7.5e-7 (grad_x), 9.0e-7 -> 9.1e-7 (grad_weight);
-//   fp32 B = 8: 309 -> 197 and 645 -> 405 us; B = 2, T = 300: 58 -> 27, 214 -> 83;
+// float64, normally distributed operands:
+//   fp32 B = 32, T = 1024, K = 768, F = 2322: errors 5.0e-7 -> 1.5e-7 (forward),
+//     8.6e-7 -> 2.5e-7 (grad_x), 9.0e-7 -> 4.5e-7 (grad_weight);
+//   the same with the steps' terms added to the accumulator one by one: 4.2e-7,
+//     7.5e-7, 9.1e-7 (and, B = 8, forward 177, both gradients 383 us);
+//   fp32 B = 8: 265 -> 187 and 617 -> 420 us; B = 2, T = 16: 57.6 -> 19.3, 179 -> 70;
+//     M = 300 with K = 1 / 16: 2.5e-8 and 7.5e-8 as before;
 //   bf16 B = 20, T = 1501, K = 768, F = 2322: 971 -> 194 us (551 TFLOP/s), 3265
 //     -> 408 us (524); B = 5, T = 1501, K = 512, F = 1040: 117 -> 25, 328 -> 75.
-// What bounds the fp32 form: the matrix cores are busy 65% of the cycles (32
+// What bounds the fp32 form: the matrix cores, busy about 65% of the cycles (32
 // per MFMA, counted) at the clock that random operands leave; halving the
 // conversion's instructions gained 3%.
 //
@@ -319,21 +327,91 @@ struct SplitStager {
   }
 };
 
-// One k-step [k0, k1) of outer index ko of the 32 x 32 block of A rows m0..,
-// B rows n0.., on the fp32 MFMA straight from memory: only for results that
-// are not finite.
-__device__ __forceinline__ void split_block_f32(const SplitOperand<float>& a,
-                                                const SplitOperand<float>& b, int m0, int n0,
-                                                int ko, int k0, int k1, int lane,
-                                                f32x16_t& acc) {
-  const int m = m0 + (lane & 31), n = n0 + (lane & 31);
-  for (int kk = k0; kk < k1; kk += 2) {
-    const int k = kk + (lane >> 5);
-    float x = 0.0f, y = 0.0f;
-    if (k < k1 && m < a.rows) x = a.p[m * a.sr + ko * a.sko + k * a.ski];
-    if (k < k1 && n < b.rows) y = b.p[n * b.sr + ko * b.sko + k * b.ski];
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc, 0, 0, 0);
+// WB neighbouring blocks of 32 x 32 (A rows m0.., B rows n0..) over the whole
+// steps [w0, w1) and the ends of the outer indices [t0, t1), on the fp32
+// MFMA straight from memory: where a result is not finite, and for reductions too
+// short to split.  Which four of eight consecutive k a lane holds is free, as long
+// as it is the same in A and B: each half of the wavefront reads four consecutive
+// ones (KC: one 16-byte load), eight k ahead of the MFMAs.  Rows past the operand
+// read its last one (unused).
+template <int L>
+__device__ __forceinline__ void split_f32_load(const SplitOperand<float>& op, const float* p,
+                                               float (&o)[4]) {
+  if constexpr (L == kSplitKC) {
+    const u32x4a4_t v = *reinterpret_cast<const u32x4a4_t*>(p);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = __uint_as_float(v[i]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = p[i * op.ski];
   }
+}
+
+template <int LA, int LB, int WB, int BK>
+__device__ __forceinline__ void split_blocks_f32(const SplitOperand<float>& oa,
+                                                 const SplitOperand<float>& ob, int m0, int n0,
+                                                 int w0, int w1, int t0, int t1, int wpb,
+                                                 int lane, f32x16_t (&acc)[WB]) {
+  const int h = lane >> 5;
+  const float* pa = oa.p + (int64_t)min(m0 + (lane & 31), oa.rows - 1) * oa.sr;
+  const float* pb[WB];
+#pragma unroll
+  for (int b = 0; b < WB; ++b) {
+    pb[b] = ob.p + (int64_t)min(n0 + 32 * b + (lane & 31), ob.rows - 1) * ob.sr;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[b][v] = 0.0f;
+  }
+  auto mfma = [&](int b, float x, float y) {
+    acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc[b], 0, 0, 0);
+  };
+  if (w1 > w0) {
+    int ko = w0 / wpb, k = (w0 - ko * wpb) * BK;
+    float x[2][4], y[2][WB][4];
+    auto load = [&](auto setc) {
+      constexpr int set = decltype(setc)::value;
+      const int64_t fa = ko * oa.sko + (k + 4 * h) * oa.ski;
+      const int64_t fb = ko * ob.sko + (k + 4 * h) * ob.ski;
+      split_f32_load<LA>(oa, pa + fa, x[set]);
+#pragma unroll
+      for (int b = 0; b < WB; ++b) split_f32_load<LB>(ob, pb[b] + fb, y[set][b]);
+    };
+    auto mfmas = [&](auto setc) {
+      constexpr int set = decltype(setc)::value;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int b = 0; b < WB; ++b) mfma(b, x[set][i], y[set][b][i]);
+    };
+    using S0 = std::integral_constant<int, 0>;
+    using S1 = std::integral_constant<int, 1>;
+    const int groups = (w1 - w0) * (BK / 8);  // of 8 k: an even number
+    auto next = [&](int g) {
+      if (g + 1 < groups) {  // (else the last group again, unused)
+        k += 8;
+        if (k == wpb * BK) {
+          k = 0;
+          ++ko;
+        }
+      }
+    };
+    load(S0{});
+    for (int g = 0; g < groups; g += 2) {
+      next(g);
+      load(S1{});
+      mfmas(S0{});
+      next(g + 1);
+      load(S0{});
+      mfmas(S1{});
+    }
+  }
+  for (int ko = t0; ko < t1; ++ko)
+    for (int kk = wpb * BK; kk < oa.kin; kk += 2) {
+      const int k = kk + h;
+      const float x = k < oa.kin ? pa[ko * oa.sko + k * oa.ski] : 0.0f;
+#pragma unroll
+      for (int b = 0; b < WB; ++b)
+        mfma(b, x, k < oa.kin ? pb[b][ko * ob.sko + k * ob.ski] : 0.0f);
+    }
 }
 
 // WB x WB blocks of 32 x 32 per wavefront: tiles of R = 64 WB rows of A and of B.
@@ -389,30 +467,48 @@ gemm_split_kernel(const SplitArgs g) {
   auto mfmas = [&](int cur) {
 #pragma unroll
     for (int t = 0; t < BK / 16; ++t) {
-      bf16x8_t fa[NP][WB], fb[NP][WB];
+      bf16x8_t fb[NP][WB];
 #pragma unroll
       for (int p = 0; p < NP; ++p)
 #pragma unroll
-        for (int a = 0; a < WB; ++a) {
-          fa[p][a] = StA::frag(lds_a[cur] + p * kPlane, wm + 32 * a, t, lane);
-          fb[p][a] = StB::frag(lds_b[cur] + p * kPlane, wn + 32 * a, t, lane);
-        }
-      auto term = [&](int pa, int pb) {
+        for (int b = 0; b < WB; ++b)
+          fb[p][b] = StB::frag(lds_b[cur] + p * kPlane, wn + 32 * b, t, lane);
 #pragma unroll
-        for (int a = 0; a < WB; ++a)
+      for (int a = 0; a < WB; ++a) {
+        bf16x8_t fa[NP];
 #pragma unroll
-          for (int b = 0; b < WB; ++b)
+        for (int p = 0; p < NP; ++p)
+          fa[p] = StA::frag(lds_a[cur] + p * kPlane, wm + 32 * a, t, lane);
+#pragma unroll
+        for (int b = 0; b < WB; ++b) {
+          if constexpr (NP == 3) {
+            // the step's sum by itself, smallest terms first, then one rounding
+            // into the accumulator
+            f32x16_t s;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) s[v] = 0.0f;
+            constexpr int kTerms[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+            static_for<6>([&](auto tc) {
+              constexpr int pa = kTerms[decltype(tc)::value][0];
+              constexpr int pb = kTerms[decltype(tc)::value][1];
+              s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[pa], fb[pb][b], s, 0, 0, 0);
+            });
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+              float x = fmaf(s[v], kSplitUnscale, acc[a][b][v]);
+              // (here, not sunk past the next branch with all of s alive)
+              asm volatile("" : "+v"(x));
+              acc[a][b][v] = x;
+            }
+          } else {
             acc[a][b] =
-                __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[pa][a], fb[pb][b], acc[a][b], 0, 0, 0);
-      };
-      if constexpr (NP == 3) {
-        term(2, 0);
-        term(0, 2);
-        term(1, 1);
-        term(1, 0);
-        term(0, 1);
+                __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[0], fb[0][b], acc[a][b], 0, 0, 0);
+          }
+        }
+        // (three pieces: holds the next row block's fragments back, whose
+        // registers are not there)
+        if constexpr (NP == 3) __builtin_amdgcn_sched_barrier(0);
       }
-      term(0, 0);
     }
   };
   SplitRaw<TI, R> ra[2], rb[2];
@@ -425,7 +521,12 @@ gemm_split_kernel(const SplitArgs g) {
   const int w0 = split * g.split_whole, w1 = min(g.KO * wpb, w0 + g.split_whole);
   const bool rows_ok = (LA != kSplitRC || g.M >= 8) && (LB != kSplitRC || g.N >= 8);
   const int np = rows_ok && w1 > w0 ? (w1 - w0) & ~1 : 0;
-  if (np > 0) {
+  // fp32: the whole tile on the fp32 MFMA, for reductions of up to 16 indices.
+  // (K = 1 on the bf16 MFMA: up to 1.5e-7 of the product, against 6e-8 rounded
+  // once; K = 2 3.4e-8 of the result in 2-norm against 3.1e-8; K = 4 3.2e-8 against
+  // 4.0e-8, but 7.6e-8 against 8e-9 for K = 7 equal products)
+  const bool direct = NP == 3 && (int64_t)g.KO * g.kin <= 16;
+  if (np > 0 && !direct) {
     int ko = w0 / wpb, ki = w0 - ko * wpb, left = np;
     int64_t offa[2], offb[2];
     auto load = [&](auto setc) {
@@ -478,63 +579,50 @@ gemm_split_kernel(const SplitArgs g) {
   const int tails = wpb * BK < g.kin ? g.KO : 0;
   const int t0 = split * g.split_tail, t1 = min(tails, t0 + g.split_tail);
   const int nodd = w1 - w0 - np, ntail = t1 - t0;
-  for (int s = 0; s < (nodd > 0 ? nodd : 0) + (ntail > 0 ? ntail : 0); ++s) {
+  for (int s = 0; s < (direct ? 0 : (nodd > 0 ? nodd : 0) + (ntail > 0 ? ntail : 0)); ++s) {
     const bool whole = s < nodd;
     const int w = w0 + np + s;
     const int ko = whole ? w / wpb : t0 + s - (nodd > 0 ? nodd : 0);
     checked(ko, whole ? (w - ko * wpb) * BK : wpb * BK);
   }
 
+  TO* C = reinterpret_cast<TO*>(g.C) + (int64_t)batch * g.scb + (int64_t)split * g.scs;
+  // lane l of a block at (mb, nb) holds column nb + l % 32 and rows
+  // mb + 8 (v / 4) + 4 (l / 32) + v % 4
+  auto store_block = [&](int mb, int nb, const f32x16_t& c) {
+    const int n = nb + (lane & 31);
+    if (n >= g.N) return;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int m = mb + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+      if (m < g.M) io_traits<TO>::store(C + (int64_t)m * g.scm + (int64_t)n * g.scn, c[v]);
+    }
+  };
   if constexpr (NP == 3) {
-    bool bad = false;
+    bool bad = direct;
 #pragma unroll
     for (int a = 0; a < WB; ++a)
 #pragma unroll
       for (int b = 0; b < WB; ++b)
 #pragma unroll
         for (int v = 0; v < 16; ++v) bad = bad || !(fabsf(acc[a][b][v]) < INFINITY);
-    if (__any(bad)) {
+    if (__builtin_amdgcn_readfirstlane(__any(bad))) {
+#pragma unroll 1
+      for (int a = 0; a < WB; ++a) {
+        f32x16_t c[WB];
+        split_blocks_f32<LA, LB, WB, BK>(oa, ob, m0 + wm + 32 * a, n0 + wn, w0, w1, t0, t1, wpb,
+                                         lane, c);
 #pragma unroll
-      for (int a = 0; a < WB; ++a)
-#pragma unroll
-        for (int b = 0; b < WB; ++b) {
-          f32x16_t c;
-#pragma unroll
-          for (int v = 0; v < 16; ++v) c[v] = 0.0f;
-          const int mb = m0 + wm + 32 * a, nb = n0 + wn + 32 * b;
-          for (int w = w0; w < w1; ++w) {
-            const int ko = w / wpb, k = (w - ko * wpb) * BK;
-            split_block_f32(oa, ob, mb, nb, ko, k, k + BK, lane, c);
-          }
-          for (int ko = t0; ko < t1; ++ko)
-            split_block_f32(oa, ob, mb, nb, ko, wpb * BK, g.kin, lane, c);
-          acc[a][b] = c;
-        }
-    } else {
-#pragma unroll
-      for (int a = 0; a < WB; ++a)
-#pragma unroll
-        for (int b = 0; b < WB; ++b)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) acc[a][b][v] *= kSplitUnscale;
+        for (int b = 0; b < WB; ++b) store_block(m0 + wm + 32 * a, n0 + wn + 32 * b, c[b]);
+      }
+      return;
     }
   }
-
-  // lane l of block (a, b) holds column n = 32 b + l % 32 and rows
-  // m = 32 a + 8 (v / 4) + 4 (l / 32) + v % 4
-  TO* C = reinterpret_cast<TO*>(g.C) + (int64_t)batch * g.scb + (int64_t)split * g.scs;
 #pragma unroll
   for (int a = 0; a < WB; ++a)
 #pragma unroll
-    for (int b = 0; b < WB; ++b) {
-      const int n = n0 + wn + 32 * b + (lane & 31);
-      if (n >= g.N) continue;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int m = m0 + wm + 32 * a + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-        if (m < g.M) io_traits<TO>::store(C + (int64_t)m * g.scm + (int64_t)n * g.scn, acc[a][b][v]);
-      }
-    }
+    for (int b = 0; b < WB; ++b)
+      store_block(m0 + wm + 32 * a, n0 + wn + 32 * b, acc[a][b]);
 }
 
 }  // namespace ltv

@@ -116,6 +116,59 @@ def test_f32_small_operands(e, other):
     assert bool((err <= (B * T + 1) * (2.0 ** -24 * mag + 2.0 ** -150)).all()), float((err / mag).max())
 
 
+@pytest.mark.parametrize("K", [1, 2, 3, 7, 16])
+def test_f32_short_reductions(K):
+    """Up to 16 indices: the fp32 arithmetic's bound, and for one index its value,
+    the product rounded once -- of the outputs and, over B T = K tokens, of the
+    weight's gradient."""
+    F, T = 131, 70
+    x, w, _ = _operands(1, T, K, F, torch.float32, 13)
+    w[0] = 1 + 2.0 ** -8 + 2.0 ** -17  # (all of its low pieces at their largest)
+    x[0, 0] = 1 + 2.0 ** -8 + 2.0 ** -17
+    ops = _ops().nanochat_cuda
+    out = ops.fused_linear_transpose_cuda_op(x, w)[0]
+    # tokens as the reduction: x and grad_out with K of them
+    x2, go = x[0].t().contiguous().unsqueeze(0), w.unsqueeze(0)
+    gx, gw = torch.empty_like(x2), torch.empty(F, T, device=DEV)
+    ops.fused_linear_transpose_backward_kernel(x2, torch.zeros(F, T, device=DEV), go, gx, gw)
+    want, mag = w.double() @ x[0].double().t(), w.double().abs() @ x[0].double().abs().t()
+    for got in (out, gw):
+        assert bool(((got.double() - want).abs() <= K * 2.0 ** -24 * mag).all())
+        if K == 1:
+            assert torch.equal(got, w * x[0].t())
+
+
+@pytest.mark.parametrize("B,T,K,F", [(3, 40, 17, 130), (3, 40, 96, 130), (8, 1024, 640, 258)])
+def test_f32_errors_are_those_of_fp32_sums_or_less(B, T, K, F):
+    """Worst case (K / 16 + 8) 2^-24 of the products' magnitudes, also where every
+    product has the same sign and its dropped terms at their largest; in 2-norm no
+    more than fp32 sums over pairs of products in order."""
+    def check(got, a, b, what):
+        # got = a @ b.T over the last axes
+        n = a.shape[1]
+        want, mag = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+        assert bool(((got.double() - want).abs() <= (n / 16 + 8) * 2.0 ** -24 * mag).all()), what
+        seq = torch.zeros_like(want, dtype=torch.float32)
+        for k in range(0, n, 2):
+            seq += a[:, k:k + 2] @ b[:, k:k + 2].t()
+        err, ref = (got.double() - want).norm(), (seq.double() - want).norm()
+        assert float(err) <= float(ref) or float(err) <= 2.0 ** -24 * float(want.norm()), what
+
+    ops = _ops().nanochat_cuda
+    for const in (False, True):
+        x, w, go = _operands(B, T, K, F, torch.float32, 14)
+        if const:
+            for t in (x, w, go):
+                t.fill_(1 + 2.0 ** -8 + 2.0 ** -17)
+        gx, gw = torch.empty_like(x), torch.empty_like(w)
+        out = ops.fused_linear_transpose_cuda_op(x, w)
+        ops.fused_linear_transpose_backward_kernel(x, w, go, gx, gw)
+        xt, gt = x.reshape(B * T, K), go.transpose(1, 2).reshape(B * T, F)
+        check(out.transpose(1, 2).reshape(B * T, F), xt, w, "out")
+        check(gx.reshape(B * T, K), gt, w.t().contiguous(), "grad_x")
+        check(gw, gt.t().contiguous(), xt.t().contiguous(), "grad_weight")
+
+
 def test_f32_values_that_the_scale_overflows():
     """Finite operands and results past the scaled range come out as usual."""
     B, T, K, F = 2, 40, 24, 70
