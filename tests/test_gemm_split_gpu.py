@@ -52,6 +52,29 @@ def test_large_tiles_and_splits(dtype, btf, T, K, F):
     _run(40, T, K, F, dtype, btf, seed=T)
 
 
+@pytest.mark.parametrize("fill", [float("nan"), float("inf"), 2.0 ** 110])
+def test_f32_operands_past_the_split_range(fill):
+    """A tensor with no element in the range that is split."""
+    B, T, K, F = 3, 150, 64, 200
+    x, w, go = _operands(B, T, K, F, torch.float32, 6)
+    x = x.sign() * fill
+    ops = _ops().nanochat_cuda
+    out = ops.fused_linear_transpose_cuda_op(x, w)
+    gx, gw = torch.empty_like(x), torch.empty_like(w)
+    ops.fused_linear_transpose_backward_kernel(x, w, go, gx, gw)
+    xd, gd = x.double(), go.double().permute(1, 0, 2).reshape(F, B * T)
+    for got, want, mag in (
+            (out, torch.matmul(w.double().unsqueeze(0), xd.transpose(1, 2).contiguous()),
+             torch.matmul(w.double().abs().unsqueeze(0), xd.abs().transpose(1, 2).contiguous())),
+            (gw, gd @ xd.reshape(B * T, K), gd.abs() @ xd.abs().reshape(B * T, K))):
+        fin = torch.isfinite(want)
+        assert bool(fin.all()) == (fill == 2.0 ** 110)
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        assert torch.equal(got.double()[torch.isinf(want)], want[torch.isinf(want)])
+        err = (got.double() - want).abs()[fin]
+        assert bool((err <= (B * T + 4) * 2.0 ** -24 * mag[fin]).all())
+
+
 @pytest.mark.parametrize("T", [40, 1024])
 def test_f32_non_finite(T):
     """Every element of the result that an infinity, a NaN or a value past the
