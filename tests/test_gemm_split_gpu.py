@@ -52,6 +52,16 @@ def test_large_tiles_and_splits(dtype, btf, T, K, F):
     _run(40, T, K, F, dtype, btf, seed=T)
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "bf16"])
+@pytest.mark.parametrize("btf", [False, True], ids=["bft", "btf"])
+@pytest.mark.parametrize("B", [1, 13, 700])
+def test_short_inner_reductions(B, btf, dtype):
+    """grad_weight over many sequences whose lengths leave 1 to 31 indices past the
+    whole k-steps: the packed steps, in one split and in several."""
+    for T in (1, 2, 5, 15, 17, 31, 33):
+        _run(B, T, 40, 50, dtype, btf, seed=T)
+
+
 @pytest.mark.parametrize("fill", [float("nan"), float("inf"), 2.0 ** 110])
 def test_f32_operands_past_the_split_range(fill):
     """A tensor with no element in the range that is split."""
