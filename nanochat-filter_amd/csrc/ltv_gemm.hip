@@ -159,27 +159,27 @@ __device__ __forceinline__ float4 ld_stream4(const float4* p) {
 
 // p[0] + p[stride] + ... (S terms, in that order), 8 loads at a time
 __device__ __forceinline__ float4 sum_splits4(const float4* p, int S, int64_t split_stride4) {
-      float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      int s = 0;
-      for (; s + 8 <= S; s += 8) {
-        float4 v[8];
-  #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = ld_stream4(&p[(int64_t)(s + j) * split_stride4]);
-  #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          acc.x += v[j].x;
-          acc.y += v[j].y;
-          acc.z += v[j].z;
-          acc.w += v[j].w;
-        }
-      }
-      for (; s < S; ++s) {
-        const float4 v = ld_stream4(&p[(int64_t)s * split_stride4]);
-        acc.x += v.x;
-        acc.y += v.y;
-        acc.z += v.z;
-        acc.w += v.w;
-      }
+  float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  int s = 0;
+  for (; s + 8 <= S; s += 8) {
+    float4 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = ld_stream4(&p[(int64_t)(s + j) * split_stride4]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      acc.x += v[j].x;
+      acc.y += v[j].y;
+      acc.z += v[j].z;
+      acc.w += v[j].w;
+    }
+  }
+  for (; s < S; ++s) {
+    const float4 v = ld_stream4(&p[(int64_t)s * split_stride4]);
+    acc.x += v.x;
+    acc.y += v.y;
+    acc.z += v.z;
+    acc.w += v.w;
+  }
   return acc;
 }
 
