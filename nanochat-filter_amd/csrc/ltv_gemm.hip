@@ -304,6 +304,9 @@ int launch_split(int dtype_in, int dtype_out, const SplitArgs& a, int batches, i
                    (dtype_out == LTV_DTYPE_BF16 || dtype_out == LTV_DTYPE_F32)),
               LTV_ERR_UNSUPPORTED, "split GEMM: unsupported dtypes %d -> %d", dtype_in,
               dtype_out);
+  // the kernel steps by one along the axis that LA / LB say is contiguous
+  LTV_REQUIRE((LA == kSplitKC ? a.saki : a.sam) == 1 && (LB == kSplitKC ? a.sbki : a.sbn) == 1,
+              LTV_ERR_UNSUPPORTED, "split GEMM: operands need a contiguous axis");
   if (splits <= 1 && split_small(a.M, a.N, batches))
     return launch_split_wb<LA, LB, 1>(dtype_in, dtype_out, a, batches, splits, st);
   return launch_split_wb<LA, LB, 2>(dtype_in, dtype_out, a, batches, splits, st);
