@@ -828,8 +828,18 @@ __device__ __forceinline__ void st_rows(const char* bh, int Tt, int tl0, uint32_
                          (int)cvt_pk_bf16(x[4 * k + 2][v], x[4 * k + 3][v])};
       __builtin_amdgcn_raw_buffer_store_b64(d, r, o, 0, kStNormal);
     } else {
-      bst128(r, o, make_uint4(__float_as_uint(x[4 * k][v]), __float_as_uint(x[4 * k + 1][v]),
-                              __float_as_uint(x[4 * k + 2][v]), __float_as_uint(x[4 * k + 3][v])));
+      // (through a register each: the vector of four elements of x made the compiler
+      // read x as vectors before it was resolved to registers, and keep it in LDS,
+      // addressed by the workgroup's size from the dispatch packet -- a read of host
+      // memory by every workgroup: the backward of 288 sequences of T = 4 .. 64
+      // took 22.5 us, 9.7 without it)
+      uint32_t d[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        d[i] = __float_as_uint(x[4 * k + i][v]);
+        asm("" : "+v"(d[i]));
+      }
+      bst128(r, o, make_uint4(d[0], d[1], d[2], d[3]));
     }
   };
   if constexpr (RM == ROWS_EVEN) {
