@@ -1197,25 +1197,46 @@ int scan_backward_impl(int dtype, const HostView4& u, const HostView4& lg, const
       cfg.L = tu.bwd_l;
       cfg.NW = tu.bwd_nw;
     }
-    // One gate per channel in bf16: the kernel holds 8 gates per lane and step,
-    // so a whole head of 128 channels left one or two wavefronts per SIMD, each
-    // waiting for its tile's loads.  64-channel slabs in workgroups of two
-    // wavefronts give more, independent ones.  Backward at T = 1024 (before ->
-    // here, us):
-    // heads of 128, 288 / 576 / 1152 sequences 139 -> 116, 236 -> 198, 363 ->
-    // 340; heads of 64, 240 / 600 sequences 77 -> 62, 151 -> 124.  32-channel
-    // slabs cut the rows below a 128-byte line (139 / 282 / 547 us).  fp32 (4
-    // gates per lane) gains nothing: 98 -> 103, 203 -> 196, 340 -> 354 us.
-    if (gm == GATE_CHANVEC && dtype == LTV_DTYPE_BF16 && cfg.CL >= 8 && tu.bwd_l == 0) {
-      cfg = ScanCfg{8, 4, 2};
-      a.nslab = (D + 8 * V - 1) / (8 * V);
-    }
     // time chunks of whole tiles; each chunk enters with its exact gradient
     // carry from the chunk-map kernels
-    const int TW = cfg.NW * (64 / cfg.CL) * cfg.L;
-    const int nc_max = bwd_max_chunks(B, H, T);
-    const int per = (T + nc_max - 1) / nc_max;
-    a.chunk_steps = std::max(2, (per + TW - 1) / TW) * TW;
+    auto tile_steps = [](const ScanCfg& c) { return c.NW * (64 / c.CL) * c.L; };
+    auto chunk_steps = [&](const ScanCfg& c) {
+      const int TW = tile_steps(c), nc_max = bwd_max_chunks(B, H, T);
+      return std::max(2, ((T + nc_max - 1) / nc_max + TW - 1) / TW) * TW;
+    };
+    // One gate per channel in bf16: the kernel holds 8 gates per lane and step, one
+    // wavefront per SIMD.  A whole head per workgroup, or slabs of 64 channels in
+    // workgroups of two wavefronts, which are more and independent, but each starts
+    // up anew and a cut last one is idle in part: whichever has the lower count of
+    // rounds of resident workgroups x (tiles per workgroup + 0.6 for its start, as
+    // measured: 5.3 us a round of one tile, 3.4 to 4.8 a further tile, a fifth more
+    // at 128 steps); equal counts go to whole slabs.  Backward, us (whole head / slabs), heads of 128, T = 1024: 288 /
+    // 576 / 1152 sequences 139 / 116, 236 / 198, 363 / 340; T = 32: 576 sequences 17 /
+    // 23, 864 20 / 29; T = 512: 864 sequences 118 / 138.  Heads of 64, T = 512, 288
+    // sequences 44 / 36; of 256, 288 sequences, T = 512 129 / 99, T = 32 18 / 24; of
+    // 96, 1152 sequences, T = 512 180 / 210.  Wider heads keep the whole head (512, 432
+    // sequences, T = 256: 128 / 154).  32-channel slabs cut the rows below a 128-byte
+    // line (139 / 282 / 547 us at heads of 128, T = 1024).  fp32 (4 gates per lane)
+    // gains nothing: 98 -> 103, 203 -> 196, 340 -> 354 us.
+    if (gm == GATE_CHANVEC && dtype == LTV_DTYPE_BF16 && cfg.CL >= 8 && D <= 256 &&
+        tu.bwd_l == 0) {
+      auto cost = [&](const ScanCfg& c, int nslab) {
+        const int cs = chunk_steps(c), TW = tile_steps(c);
+        const int64_t wgs = (int64_t)B * H * nslab * ((T + cs - 1) / cs);
+        const int64_t slots = (int64_t)scan_cu_count() * 4 / c.NW;
+        const double tile = c.NW == 4 && c.CL == 8 ? 1.2 : 1.0;
+        return (double)((wgs + slots - 1) / slots) *
+               (tile * ((std::min(cs, T) + TW - 1) / TW) + 0.6);
+      };
+      const ScanCfg slab{8, 4, 2};
+      const int nslab = (D + 8 * V - 1) / (8 * V);
+      const double whole = cost(cfg, 1), slabs = cost(slab, nslab);
+      if (slabs < whole || (slabs == whole && D % (8 * V) == 0)) {
+        cfg = slab;
+        a.nslab = nslab;
+      }
+    }
+    a.chunk_steps = chunk_steps(cfg);
     a.nchunk = (T + a.chunk_steps - 1) / a.chunk_steps;
     const int64_t grid = (int64_t)B * H * a.nslab * a.nchunk;
     LTV_REQUIRE(grid < (1ll << 31), LTV_ERR_UNSUPPORTED, "grid too large");

@@ -4,7 +4,8 @@ workgroups per head.
 Exact integer cases where a slab can go wrong: heads of one slab, of one and a
 vector (a last slab with one lane of 8), of a slab and a half, of several, the
 widest; T of one step, one short of, at and past a tile of 64, several tiles;
-few sequences with their time cut into chunks.
+few sequences with their time cut into chunks.  Which of these run in slabs and
+which with a whole head per workgroup is the library's choice.
 """
 
 from __future__ import annotations
@@ -23,10 +24,22 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("D", [64, 72, 96, 128, 200, 256, 512])
 @pytest.mark.parametrize("T", [1, 63, 64, 65, 200, 300])
 def test_slab_backward_exact(D, T, monkeypatch):
+    _exact(2, D, T, monkeypatch)
+
+
+@pytest.mark.parametrize("D,T", [(40, 200), (64, 65), (64, 200), (72, 65), (128, 130), (200, 65),
+                                 (200, 200), (256, 65), (256, 200)])
+def test_slab_backward_many_sequences(D, T, monkeypatch):
+    """More sequences than compute units, where the slabs are chosen (two tiles and
+    more; heads of up to one slab, of several, of a cut last one)."""
+    _exact(72, D, T, monkeypatch)
+
+
+def _exact(B, D, T, monkeypatch):
     from nanochat_amd import _native as N
 
     monkeypatch.setattr(N, "chain_workspace_for", lambda *a, **k: N._NO_CHAIN)
-    B, NH, NKVH, r, dtype = 2, 2, 1, 1, torch.bfloat16
+    NH, NKVH, r, dtype = 2, 1, 1, torch.bfloat16
     H, Da = NH + 2 * NKVH, D
     c = int_combined(B, T, NH, NKVH, Da, r)
     ini, bias = int_inits(B, NH, NKVH, Da, r), int_logit_bias(NH, NKVH, Da, False)
