@@ -205,8 +205,9 @@ int ltv_hm_scan_backward(int dtype, const void* combined, const int64_t combined
  *   passed is not touched.  With many chunks per sequence NULL is the faster
  *   choice: ltv_hm_scan_backward_chain_pays(...) returns 1 where the chained
  *   kernel is, else 0.
- *   (LTV_SCAN_BWD_CHAIN_CFG="L,NW" forces it, "0" turns it off.)  `workspace` is sized by ltv_hm_scan_backward_workspace_size
- *   as before (it covers either kernel's dbias partials).
+ *   (LTV_SCAN_BWD_CHAIN_CFG="L,NW" forces it, "0" turns it off.)  `workspace`
+ *   is sized by ltv_hm_scan_backward_workspace_size as before (it covers
+ *   either kernel's dbias partials).
  *
  * Replaces the same reference backward as ltv_hm_scan_backward; the chain
  * workspace has no counterpart there (the reference walks T serially per

@@ -1473,18 +1473,21 @@ extern "C" size_t ltv_hm_scan_backward_chain_workspace_size(int dtype, int B, in
   return bwd_chain_plan(dtype, B, T, NH + 2 * NKVH, Da, r).bytes;
 }
 
-// Whether the chained backward is the faster one.  Every chunk waits for the one
-// after it, about 0.75 us, so with many chunks the tile kernel over chunk maps
-// wins: measured on MI355X in bf16 (chained / maps), 16 chunks 52 / 53 us at 144
-// sequences and 34 / 36 at 72, 64 chunks 90 / 83 at 72, 128 chunks 120 / 85 at 36.
-// With fewer than 16 sequences both are short (47 chunks of 8 sequences 42 / 29
-// us); the chained form, one launch instead of three, is kept to 48 chunks there.
+// Whether the chained backward is the faster one: up to 16 chunks per sequence.
+// Every chunk waits for the one after it, about 0.6 us, so with many chunks the tile
+// kernel over chunk maps wins: measured on MI355X, heads of 128 (chained / maps, us),
+// bf16 at 3 / 8 / 36 / 72 / 144 sequences: 12 chunks 17 / 19, 18 / 19, 23 / 21, 29 / 30,
+// 44 / 44; 16 chunks 19 / 19, 21 / 20, 27 / 26, 35 / 37, 53 / 52; 24 chunks 25 / 19, 26 /
+// 20, 34 / 31, 45 / 46, 70 / 64; 48 chunks 39 / 21, 42 / 22, 55 / 47, 73 / 65, 122 / 104;
+// fp32, 16 chunks 18 / 19, 19 / 20, 27 / 23, 33 / 30, 49 / 43.  The maps' two launches
+// more do not show in a step's host time (1 x 1280 .. 6000 tokens, 3 to 12
+// sequences: 136-140 us bf16 either way, fp32 330-377 / 324-343).
 extern "C" int ltv_hm_scan_backward_chain_pays(int dtype, int B, int T, int NH, int NKVH, int Da,
                                                int r) {
   if (check_shape(dtype, B, T, NH, NKVH, Da, r) != LTV_OK) return 0;
   const BwdChainPlan p = bwd_chain_plan(dtype, B, T, NH + 2 * NKVH, Da, r);
   if (p.bytes == 0) return 0;
-  return tuning().bwd_chain_l > 0 || p.nchunk <= (p.nseq >= 16 ? 16 : 48) ? 1 : 0;
+  return tuning().bwd_chain_l > 0 || p.nchunk <= 16 ? 1 : 0;
 }
 
 extern "C" int ltv_chain_take_error(void) {

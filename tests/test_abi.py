@@ -219,3 +219,17 @@ def test_peaks_library_exports_its_header():
     assert sorted(names) == ["ltv_peak_mfma", "ltv_peak_overlap", "ltv_peak_stream"]
     lib = ctypes.CDLL(path)
     assert all(hasattr(lib, n) for n in names)
+
+
+@pytest.mark.parametrize("B,NH", [(1, 1), (2, 2), (8, 6)])
+def test_chained_backward_is_kept_to_few_chunks(B, NH):
+    """The chained backward hands a carry from chunk to chunk; past 16 chunks of a
+    sequence the chunk maps take less time, however few the sequences."""
+    from nanochat_amd import _native as N
+
+    lib = N.lib()
+    for dtype, steps in ((1, 64), (0, 32)):  # a chunk at heads of 128: bf16, fp32
+        for chunks, pays in ((2, 1), (16, 1), (17, 0), (47, 0)):
+            T = chunks * steps
+            assert lib.ltv_hm_scan_backward_chain_workspace_size(dtype, B, T, NH, NH, 1, 128) > 0
+            assert lib.ltv_hm_scan_backward_chain_pays(dtype, B, T, NH, NH, 1, 128) == pays
