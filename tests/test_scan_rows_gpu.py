@@ -67,10 +67,26 @@ def _check(dtype, B, NH, NKVH, D, r, T, pitch, offset):
 @pytest.mark.parametrize("dtype", DTYPES, ids=io_name)
 @pytest.mark.parametrize("T", [4, 5, 6, 7, 63, 64, 65, 130, 259, 1030])
 def test_rows_few_sequences(dtype, T):
-    """Chained kernels from two chunks on, the tile kernels below."""
+    """The forward's tile kernel; the backward chained from two chunks on (up to
+    16), the tile kernels below and above."""
     for D, r in ((128, 128), (64, 16), (32, 32)):
         for pitch, offset in PITCHES:
             _check(dtype, 1, 2, 1, D, r, T, pitch, offset)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=io_name)
+@pytest.mark.parametrize("T", [3585, 4096, 4099, 4606])
+def test_rows_chained_forward(dtype, T):
+    """The chained forward, two quads of steps per lane: it takes sequences from 8
+    chunks of 512 steps on (a last chunk of one step, a whole one, one of
+    three steps, one whose last quad is cut)."""
+    from nanochat_amd import _native as N
+
+    for D, r, NH, NKVH in ((128, 128, 1, 1), (64, 16, 2, 1)):
+        assert N.lib().ltv_hm_scan_forward_chain_workspace_size(
+            N.dtype_code(dtype), 1, T, NH, NKVH, D // r, r) > 0
+        for pitch, offset in PITCHES:
+            _check(dtype, 1, NH, NKVH, D, r, T, pitch, offset)
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=io_name)
