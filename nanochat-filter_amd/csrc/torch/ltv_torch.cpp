@@ -352,7 +352,8 @@ pybind11::object decode_rows(const Tensor& x, const Tensor& wpack, const Tensor&
     st[2 * i + 1] = t.stride(1);
   }
   if (!plain(wpack) || wpack.device() != x.device() || bias.device() != x.device() ||
-      wpack.scalar_type() != at::kBFloat16)
+      wpack.scalar_type() != at::kBFloat16 || wpack.dim() != 2 || !wpack.is_contiguous() ||
+      wpack.size(0) != ltv_qkv_packed_width(H, D, Da) || wpack.size(1) != C)
     return pybind11::none();
   c10::OptionalDeviceGuard guard(x.device());
   Tensor out = at::empty({B, 1, H, D}, x.options());

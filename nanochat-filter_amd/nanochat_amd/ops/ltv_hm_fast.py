@@ -162,6 +162,9 @@ def decode_step(x: torch.Tensor, wpack: torch.Tensor, prev, logit_bias: torch.Te
         raise RuntimeError("decode_step computes in bf16")
     D = Da * r
     H = NH + 2 * NKVH
+    if tuple(wpack.shape) != (packed_width(H, D, Da), C) or not wpack.is_contiguous():
+        raise RuntimeError(f"the packed weight must be {(packed_width(H, D, Da), C)} for x of "
+                           f"width {C}, got {tuple(wpack.shape)}")
     if x_cs != 1 or x_rs % 8 != 0:
         x = x.reshape(B, C).contiguous()
         x_rs = C

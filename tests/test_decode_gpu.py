@@ -335,3 +335,23 @@ def test_decode_into_rows_declines_rows_it_cannot_store():
         assert out is not None
         torch.cuda.synchronize()
         assert torch.equal(out[0][:, 0], good[0])
+
+
+@pytest.mark.parametrize("wrong", [-64, -16, 16, 64])
+def test_decode_refuses_a_width_that_is_not_the_weights(wrong):
+    """x of another width than the packed weight's rows is refused as the
+    projection refuses it, in place and with new rows, and nothing is written."""
+    from nanochat_amd.ltv.ltv_filter import LtvInitValues
+    NH, NKVH, D, B = 2, 1, 64, 3
+    f = _make_filter(NH, NKVH, D, D, seed=5)
+    x = torch.randn(B, 1, NH * D + wrong).to(torch.bfloat16).to(DEV)
+    rows = [torch.randn(B, nh, D).to(torch.bfloat16).to(DEV) for nh in (NH, NKVH, NKVH)]
+    before = [t.clone() for t in rows]
+    prev = LtvInitValues(q=rows[0], k=rows[1], v=rows[2])
+    with torch.no_grad():
+        with pytest.raises(RuntimeError, match="packed weight"):
+            f.decode_into_rows(x, prev, tuple(rows))
+        with pytest.raises(RuntimeError, match="packed weight"):
+            f(x, prev)
+    for t, t0 in zip(rows, before):
+        assert torch.equal(t, t0)
