@@ -473,14 +473,15 @@ LtSplits lt_splits(int M, int K, int F) {
 }
 
 // grad_weight's split over the B T reduction on the split GEMM.  With `slots`
-// workgroups resident at once (kSplitWgPerCu per CU) and `tiles` 128 x 128
+// workgroups resident at once (SplitTraits) and `tiles` 128 x 128
 // output tiles, S splits take ceil(tiles S / slots) rounds of 1 / S of the
 // reduction each: S minimises rounds / S (the smallest S within 4% of the best,
 // up to 32 splits of at least 256 indices).  S = 1 needs no workspace.
-int lt_split_splits(int B, int T, int K, int F) {
+int lt_split_splits(int dtype, int B, int T, int K, int F) {
   const int64_t M = (int64_t)B * T;
   const int64_t tiles = std::max<int64_t>(1, (int64_t)((K + 127) / 128) * ((F + 127) / 128));
-  const int slots = kSplitWgPerCu * device_cu_count();
+  const int slots = device_cu_count() * (dtype == LTV_DTYPE_F32 ? SplitTraits<float>::kWgPerCu
+                                                                : SplitTraits<bf16_t>::kWgPerCu);
   auto cost = [&](int s) { return (double)((tiles * s + slots - 1) / slots) / s; };
   double best = cost(1);
   int smax = 1;
@@ -502,8 +503,8 @@ bool lt_backward_pointers_ok(const void* x, const void* weight, const void* grad
          (grad_weight || nw == 0) && (grad_out || ng == 0);
 }
 
-size_t lt_split_workspace(int B, int T, int K, int F) {
-  const int S = lt_split_splits(B, T, K, F);
+size_t lt_split_workspace(int dtype, int B, int T, int K, int F) {
+  const int S = lt_split_splits(dtype, B, T, K, F);
   return S > 1 ? (size_t)S * F * K * sizeof(float) : 0;
 }
 
@@ -538,8 +539,8 @@ int lt_backward_split(int dtype, const void* x, const void* weight, const void* 
     return btf ? launch_split<kSplitRC, kSplitRC>(dtype, dtype_out, w, 1, S, st)
                : launch_split<kSplitKC, kSplitRC>(dtype, dtype_out, w, 1, S, st);
   };
-  const int S = lt_split_splits(B, T, K, F);
-  const size_t need = lt_split_workspace(B, T, K, F);
+  const int S = lt_split_splits(dtype, B, T, K, F);
+  const size_t need = lt_split_workspace(dtype, B, T, K, F);
   if (need == 0 || workspace == nullptr || workspace_bytes < need) return launch_w(dtype, 1);
   w.C = workspace;
   w.scs = (int64_t)F * K;
@@ -568,7 +569,8 @@ extern "C" int ltv_linear_transpose_backward(int dtype, const void* x, const voi
 extern "C" size_t ltv_linear_transpose_backward_workspace_size(int dtype, int B, int T, int K,
                                                                 int F, int grad_out_is_btf) {
   if (B <= 0 || T <= 0 || K <= 0 || F <= 0) return 0;
-  if (!lt_backward_mfma(dtype, grad_out_is_btf, B, T, K, F)) return lt_split_workspace(B, T, K, F);
+  if (!lt_backward_mfma(dtype, grad_out_is_btf, B, T, K, F))
+    return lt_split_workspace(dtype, B, T, K, F);
   const LtSplits p = lt_splits(B * T, K, F);
   return (size_t)p.S * p.Fr * K * sizeof(float);
 }

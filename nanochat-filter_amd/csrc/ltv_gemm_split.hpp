@@ -12,12 +12,12 @@
 // subnormal pieces lose no bits either: kSplitScale), and a
 // product is six MFMA terms, smallest first: x3 y1, x1 y3, x2 y2, x2 y1, x1 y2,
 // x1 y1.  The three left out come to at most 2^-24 of a product (x2 y3 and x3 y2
-// 2^-25 each), 2^-27.5 in the mean.  The bf16 MFMA does not round its sums
-// correctly: of two addends the smaller is cut below the last bit of the larger.
-// So the terms of a step of 16 indices are summed by themselves, from zero, and a
-// step's sum enters the accumulator with one fp32 rounding: K / 16 of them, where
-// the fp32 MFMA takes K / 2.  Worst case (K / 16 + 8) 2^-24 of the sum of the
-// products' magnitudes; reductions of up to 16 indices, where that is more than
+// 2^-25 each), 2^-27.5 in the mean.  The bf16 MFMA rounds its sums correctly where
+// the accumulator is the largest addend, and cuts addends below the last bit of the
+// largest elsewhere.  So x1 y1 has an accumulator to itself, with K / 16 roundings
+// where the fp32 MFMA takes K / 2, and the five smaller terms (2^-8 of it) share
+// another; they are added at the end.  Worst case (K / 16 + 8) 2^-24 of the sum of
+// the products' magnitudes; reductions of up to 16 indices, where that is more than
 // the fp32 arithmetic's K 2^-24, run on the fp32 MFMA (split_blocks_f32).
 // A bf16 MFMA term is 16 times as fast as the fp32 MFMA (2.5 against 0.157
 // PFLOP/s nominal), six of them 2.7 times.  Non-finite results send the
@@ -25,18 +25,17 @@
 // no such split, nor has a value that the scale takes past the largest bf16), so
 // infinities and NaNs come out as fp32 arithmetic gives them; a tile that meets
 // one in its first step goes there at once.  (B = 8, T = 1024, K = 768, F = 2322,
-// all NaN: forward 342, both gradients 902 us, against 265 and 617 for the fp32
-// MFMA kernel; one NaN 283 and 526.)
+// all NaN: forward 393, both gradients 884 us, against 265 and 617 for the fp32
+// MFMA kernel; one NaN 289 and 484.)
 // bf16 operands are one piece: the products are exact, as they always were.
 //
 // Measured on MI355X against the fp32-MFMA kernel before it (128 x 128 tiles,
 // quads, one element per load off a 16-byte boundary), 2-norm errors against
 // float64, normally distributed operands:
-//   fp32 B = 32, T = 1024, K = 768, F = 2322: errors 5.0e-7 -> 1.5e-7 (forward),
-//     8.6e-7 -> 2.5e-7 (grad_x), 9.0e-7 -> 4.5e-7 (grad_weight);
-//   the same with the steps' terms added to the accumulator one by one: 4.2e-7,
-//     7.5e-7, 9.1e-7 (and, B = 8, forward 177, both gradients 383 us);
-//   fp32 B = 8: 265 -> 187 and 617 -> 420 us; B = 2, T = 16: 57.6 -> 19.3, 179 -> 70;
+//   fp32 B = 32, T = 1024, K = 768, F = 2322: errors 5.0e-7 -> 1.6e-7 (forward),
+//     8.6e-7 -> 2.9e-7 (grad_x), 9.0e-7 -> 3.1e-7 (grad_weight); with all six terms in
+//     one accumulator 4.2e-7, 7.5e-7, 9.1e-7 (B = 8 of it 177 and 383 us);
+//   fp32 B = 8: 265 -> 185 and 617 -> 388 us; B = 2, T = 16: 57.6 -> 16, 179 -> 60;
 //     M = 300 with K = 1 / 16: 2.5e-8 and 7.5e-8 as before;
 //   bf16 B = 20, T = 1501, K = 768, F = 2322: 971 -> 194 us (551 TFLOP/s), 3265
 //     -> 408 us (524); B = 5, T = 1501, K = 512, F = 1040: 117 -> 25, 328 -> 75.
@@ -44,9 +43,12 @@
 // per MFMA, counted) at the clock that random operands leave; halving the
 // conversion's instructions gained 3%.
 //
-// 128 x 128 output tiles, 4 wavefronts of 64 x 64, three workgroups per CU
-// (three wavefronts per SIMD, so that one's barrier, load wait or conversion
-// leaves the matrix core to the others); 64 x 64 tiles where those are too few.
+// 128 x 128 output tiles, 4 wavefronts of 64 x 64, three workgroups per CU in bf16
+// and two in fp32 (so that one wavefront's barrier, load wait or conversion leaves
+// the matrix core to the SIMD's others; fp32's second accumulator takes the
+// registers of a third: with one accumulator, each step's terms summed from zero and
+// added to it, three fit, but the additions cost more: 197 and 443 us against 190
+// and 404); 64 x 64 tiles where those are too few.
 // The global loads run two steps ahead in registers, and the next step is
 // converted into the other of two LDS stages while this one runs its MFMAs; one
 // barrier per step.
@@ -64,8 +66,8 @@
 // Whole steps never straddle an outer index: each ko has kin / BK of them, and where
 // kin is not a multiple, its last indices go into steps of their own, packed over
 // the outer indices (read element by element).  A step for each of them is up to 16
-// times the work: both gradients of B = 64, T = 5, K = 128, F = 390 147 us in fp32
-// (80 before this kernel), packed 60; bf16 76 -> 39.  A workgroup runs its whole steps first, pipelined, then
+// times the work: grad_weight of many short sequences, B = 64, T = 5, K = 128, F =
+// 390 in fp32, both gradients 147 -> 60 us, bf16 76 -> 39.  A workgroup runs its whole steps first, pipelined, then
 // the packed ones.  Split-K: blockIdx.z =
 // batch * splits + split; split s takes the whole steps [s split_whole,
 // (s + 1) split_whole) and the last indices of the outer indices [s split_tail,
@@ -81,7 +83,6 @@ namespace ltv {
 enum SplitLayout { kSplitKC = 0, kSplitRC = 1 };
 
 constexpr int kSplitThreads = 256;  // 4 wavefronts, 2 x 2
-constexpr int kSplitWgPerCu = 3;
 
 // fp32 operands are split at 2^24 times their value: the last bit of the
 // smallest subnormal then lies at 2^-125, so every piece of every operand is a
@@ -95,6 +96,7 @@ constexpr float kSplitUnscale = 1.0f / (kSplitScale * kSplitScale);
 template <typename TI>
 struct SplitTraits {
   static constexpr int kPieces = sizeof(TI) == 4 ? 3 : 1;
+  static constexpr int kWgPerCu = sizeof(TI) == 4 ? 2 : 3;  // of 128 x 128 tiles
   __host__ __device__ static constexpr int bk(int R) { return sizeof(TI) == 4 && R == 128 ? 16 : 32; }
 };
 
@@ -450,7 +452,7 @@ __device__ __forceinline__ void split_blocks_f32(const SplitOperand<float>& oa,
 
 // WB x WB blocks of 32 x 32 per wavefront: tiles of R = 64 WB rows of A and of B.
 template <typename TI, typename TO, int LA, int LB, int WB>
-__global__ void __launch_bounds__(kSplitThreads, kSplitWgPerCu)
+__global__ void __launch_bounds__(kSplitThreads, WB == 2 ? SplitTraits<TI>::kWgPerCu : 3)
 gemm_split_kernel(const SplitArgs g) {
   constexpr int R = 64 * WB;
   using StA = SplitStager<TI, LA, R>;
@@ -493,6 +495,16 @@ gemm_split_kernel(const SplitArgs g) {
     for (int b = 0; b < WB; ++b)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
+  // fp32: the sums of the terms below x1 y1
+  f32x16_t low[NP == 3 ? WB : 1][NP == 3 ? WB : 1];
+  if constexpr (NP == 3) {
+#pragma unroll
+    for (int a = 0; a < WB; ++a)
+#pragma unroll
+      for (int b = 0; b < WB; ++b)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) low[a][b][v] = 0.0f;
+  }
 
   StA sa;
   StB sb;
@@ -516,32 +528,18 @@ gemm_split_kernel(const SplitArgs g) {
 #pragma unroll
         for (int b = 0; b < WB; ++b) {
           if constexpr (NP == 3) {
-            // the step's sum by itself, smallest terms first, then one rounding
-            // into the accumulator
-            f32x16_t s;
-#pragma unroll
-            for (int v = 0; v < 16; ++v) s[v] = 0.0f;
-            constexpr int kTerms[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
-            static_for<6>([&](auto tc) {
+            // smallest terms first; x1 y1 by itself
+            constexpr int kTerms[5][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}};
+            static_for<5>([&](auto tc) {
               constexpr int pa = kTerms[decltype(tc)::value][0];
               constexpr int pb = kTerms[decltype(tc)::value][1];
-              s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[pa], fb[pb][b], s, 0, 0, 0);
+              low[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[pa], fb[pb][b], low[a][b],
+                                                                  0, 0, 0);
             });
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-              float x = fmaf(s[v], kSplitUnscale, acc[a][b][v]);
-              // (here, not sunk past the next branch with all of s alive)
-              asm volatile("" : "+v"(x));
-              acc[a][b][v] = x;
-            }
-          } else {
-            acc[a][b] =
-                __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[0], fb[0][b], acc[a][b], 0, 0, 0);
           }
+          acc[a][b] =
+              __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[0], fb[0][b], acc[a][b], 0, 0, 0);
         }
-        // (three pieces: holds the next row block's fragments back, whose
-        // registers are not there)
-        if constexpr (NP == 3) __builtin_amdgcn_sched_barrier(0);
       }
     }
   };
@@ -643,6 +641,12 @@ gemm_split_kernel(const SplitArgs g) {
     }
   };
   if constexpr (NP == 3) {
+#pragma unroll
+    for (int a = 0; a < WB; ++a)
+#pragma unroll
+      for (int b = 0; b < WB; ++b)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[a][b][v] = (acc[a][b][v] + low[a][b][v]) * kSplitUnscale;
     bool bad = direct;
 #pragma unroll
     for (int a = 0; a < WB; ++a)
