@@ -161,7 +161,8 @@ struct SplitStager {
 
   // chunk c at ko = 0, k0 = 0.  Rows past the operand: row 0.  An RC chunk that
   // the operand's end cuts is read `early` rows early, to end with it, and
-  // shifted into place when it is stored.
+  // shifted into place when it is stored; with fewer rows than a chunk it is read
+  // on into the next k's rows, whose results are not stored.
   const TI* rp[NC];
   uint32_t early;
 
@@ -178,7 +179,7 @@ struct SplitStager {
   __device__ __forceinline__ void setup(const SplitOperand<TI>& op) {
     // (an RC thread's chunks share their rows)
     const int over = op.row0 + row_of(0) + 8 - op.rows;
-    early = L == kSplitRC && over > 0 && over < 8 ? (uint32_t)over : 0u;
+    early = L == kSplitRC && over > 0 && over < 8 && op.rows >= 8 ? (uint32_t)over : 0u;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const int row = op.row0 + row_of(c);
@@ -551,8 +552,11 @@ gemm_split_kernel(const SplitArgs g) {
   // the last step is loaded and stored again, unused: no branch in the loop.
   const int wpb = g.kin / BK;  // whole steps per outer index
   const int w0 = split * g.split_whole, w1 = min(g.KO * wpb, w0 + g.split_whole);
-  const bool rows_ok = (LA != kSplitRC || g.M >= 8) && (LB != kSplitRC || g.N >= 8);
-  const int np = rows_ok && w1 > w0 ? (w1 - w0) & ~1 : 0;
+  // (an RC operand with fewer rows than a chunk is read past its row: every step but
+  // the reduction's last whole one has at least BK more k behind it)
+  const bool few = (LA == kSplitRC && g.M < 8) || (LB == kSplitRC && g.N < 8);
+  const int ahead = w1 - w0 - (few && w1 == g.KO * wpb ? 1 : 0);
+  const int np = ahead > 0 ? ahead & ~1 : 0;
   // fp32: the whole tile on the fp32 MFMA, for reductions of up to 16 indices.
   // (K = 1 on the bf16 MFMA: up to 1.5e-7 of the product, against 6e-8 rounded
   // once; K = 2 3.4e-8 of the result in 2-norm against 3.1e-8; K = 4 3.2e-8 against
@@ -600,8 +604,8 @@ gemm_split_kernel(const SplitArgs g) {
   }
   const int tail = g.kin - wpb * BK, tails = tail > 0 ? g.KO : 0;
   const int t0 = split * g.split_tail, t1 = min(tails, t0 + g.split_tail);
-  // The steps left: an odd whole one (all of them where an RC operand has fewer
-  // rows than a chunk), then the ends of the outer indices' ranges, packed.
+  // The steps left: the last whole ones, then the ends of the outer indices' ranges,
+  // packed.
   if (!direct) {
     int tko = t0, tr = 0;
     int64_t left = (int64_t)(t1 - t0) * tail;
