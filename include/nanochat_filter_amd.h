@@ -395,8 +395,9 @@ int ltv_hm_look_back_scan_backward_split_ws(
  * bf16 MFMA (fp32 accumulation) and writes the (B, F, T) layout directly; fp32
  * and the other bf16 shapes run on a strided GEMM (each fp32 operand as three
  * bf16 pieces, six bf16 MFMA terms per product, fp32 accumulation; any sizes
- * and alignment).  x and weight may be NULL when
- * K = 0 (out is then zeros).
+ * and alignment, any magnitudes; operands from 2^104 and sums from 2^80 on,
+ * infinities and NaNs on the fp32 MFMA, at a lower rate).  x and weight may
+ * be NULL when K = 0 (out is then zeros).
  * Replaces fused_linear_transpose (cpp_ewma/src/fused_linear_transpose_forward.cu:23-58,
  * called from nanochat/ops/fused_linear_transpose.py:20-40).
  * ---------------------------------------------------------------------- */

@@ -12,13 +12,14 @@
 // subnormal pieces lose no bits either: kSplitScale), and a
 // product is six MFMA terms, smallest first: x3 y1, x1 y3, x2 y2, x2 y1, x1 y2,
 // x1 y1.  The three left out come to at most 2^-24 of a product (x2 y3 and x3 y2
-// 2^-25 each), 2^-27.5 in the mean.  The bf16 MFMA rounds its sums correctly where
-// the accumulator is the largest addend, and cuts addends below the last bit of the
-// largest elsewhere.  So x1 y1 has an accumulator to itself, with K / 16 roundings
-// where the fp32 MFMA takes K / 2, and the five smaller terms (2^-8 of it) share
-// another; they are added at the end.  Worst case (K / 16 + 8) 2^-24 of the sum of
-// the products' magnitudes; reductions of up to 16 indices, where that is more than
-// the fp32 arithmetic's K 2^-24, run on the fp32 MFMA (split_blocks_f32).
+// 2^-25 each), 2^-27.5 in the mean.  The bf16 MFMA was seen to round correctly
+// where the accumulator is the largest addend, and to cut addends below the last bit
+// of the largest elsewhere.  So x1 y1 has an accumulator to itself, with K / 16
+// roundings where the fp32 MFMA takes K / 2, and the five smaller terms (2^-8 of it)
+// share another; they are added at the end.  Worst case, with every cut bit set,
+// (K / 15 + 18) 2^-24 of the sum of the products' magnitudes, against K 2^-24 in
+// fp32 arithmetic; reductions of up to 16 indices, which show the cut bits, run on
+// the fp32 MFMA (split_blocks_f32).
 // A bf16 MFMA term is 16 times as fast as the fp32 MFMA (2.5 against 0.157
 // PFLOP/s nominal), six of them 2.7 times.  Non-finite results send the
 // wavefront's part of the tile through the fp32 MFMA too (an infinity has
@@ -39,9 +40,9 @@
 //     M = 300 with K = 1 / 16: 2.5e-8 and 7.5e-8 as before;
 //   bf16 B = 20, T = 1501, K = 768, F = 2322: 971 -> 194 us (551 TFLOP/s), 3265
 //     -> 408 us (524); B = 5, T = 1501, K = 512, F = 1040: 117 -> 25, 328 -> 75.
-// What bounds the fp32 form: the matrix cores, busy about 65% of the cycles (32
-// per MFMA, counted) at the clock that random operands leave; halving the
-// conversion's instructions gained 3%.
+// What bounds the fp32 form: the matrix cores, busy half of the cycles (32 per MFMA,
+// counted) at the clock that random operands leave, and the conversion beside them;
+// halving its instructions gained 3%.
 //
 // 128 x 128 output tiles, 4 wavefronts of 64 x 64, three workgroups per CU in bf16
 // and two in fp32 (so that one wavefront's barrier, load wait or conversion leaves
@@ -65,13 +66,13 @@
 //
 // Whole steps never straddle an outer index: each ko has kin / BK of them, and where
 // kin is not a multiple, its last indices go into steps of their own, packed over
-// the outer indices (read element by element).  A step for each of them is up to 16
-// times the work: grad_weight of many short sequences, B = 64, T = 5, K = 128, F =
-// 390 in fp32, both gradients 147 -> 60 us, bf16 76 -> 39.  A workgroup runs its whole steps first, pipelined, then
-// the packed ones.  Split-K: blockIdx.z =
-// batch * splits + split; split s takes the whole steps [s split_whole,
-// (s + 1) split_whole) and the last indices of the outer indices [s split_tail,
-// (s + 1) split_tail), and sums them into C + s scs.
+// the outer indices (read element by element).  A step for each ko's would be up to
+// 16 times the work: grad_weight of many short sequences, B = 64, T = 5, K = 128, F =
+// 390 in fp32, both gradients 147 -> 60 us, bf16 76 -> 39.  A workgroup runs its
+// whole steps first, pipelined, then the packed ones.  Split-K: blockIdx.z = batch *
+// splits + split; split s takes the whole steps [s split_whole, (s + 1) split_whole)
+// and the last indices of the outer indices [s split_tail, (s + 1) split_tail), and
+// sums them into C + s scs.
 #pragma once
 
 #include "ltv_gemm_dma.hpp"

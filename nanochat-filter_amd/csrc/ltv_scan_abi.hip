@@ -322,13 +322,14 @@ inline bool vec_ok(const void* p, const int64_t* s, int nd_outer, int V) {
 // to 32 channel lanes and at least one quad of steps (T >= 4).  ROWS_EVEN:
 // rows of whole quads that start on a dword; ROWS_ANY: any other T or
 // alignment.  Element by element -- the only other way to read such a view --
-// measured slower everywhere (MI355X kernel times, element / row modes):
+// measured slower, or at T < 16 equal within 1 us in 15 (MI355X kernel times,
+// element / row modes):
 //   bf16, B = 16, T = 1024, 18 heads of 128, one gate (ROWS_EVEN): forward
 //     103.2 / 36.6 us (4.1 TB/s), backward 365 / 88 us (2.6 TB/s);
 //   bf16, B = 5, T = 1501, 16 heads of 64 (ROWS_ANY): forward 49.9 / 26.2 us,
 //     backward 136 us in time chunks / 31.3 us chained;
 //   fp32, B = 8, T = 1024, 18 heads of 128 (ROWS_EVEN): forward 55.1 / 32.3 us,
-//     backward 225 us in time chunks / 92 us chained.
+//     backward 225 / 85 us in time chunks.
 int rows_mode(int dtype, const void* p, const int64_t* s, int T, int D, int r) {
   const int V = dtype == LTV_DTYPE_BF16 ? 8 : 4;
   if (s[2] != 1 || T < 4 || r % V != 0) return ROWS_NONE;  // (r % V == 0: so is D)
