@@ -206,8 +206,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> forward_impl(
 
 variable_list backward_impl(const variable_list& saved, const variable_list& grads,
                             const Spec& c) {
-  const Tensor &x = saved[0], &wpack = saved[1], &values = saved[2], &logits = saved[3],
-               &inits = saved[4], &bias = saved[5];
+  // (a saved-tensor hook may hand x and the scan's tensors back in another layout)
+  const Tensor x = saved[0].contiguous();
+  const Tensor &wpack = saved[1], &values = saved[2], &logits = saved[3], &inits = saved[4],
+               &bias = saved[5];
   c10::OptionalDeviceGuard guard(x.device());
   void* st = current_stream(x);
   const int H = c.H(), D = c.D(), F = c.F();
@@ -232,7 +234,8 @@ variable_list backward_impl(const variable_list& saved, const variable_list& gra
     bytes = ltv_hm_scan_backward_chain_workspace_size(LTV_DTYPE_BF16, c.B, c.T, c.NH, c.NKVH,
                                                       c.Da, c.r);
   const Tensor cw = chain_workspace(x, st, bytes);
-  const Strides vs(values), ls(logits.stride(0), c.Da, logits.stride(1), 1),
+  const Strides vs(values),
+      ls(logits.stride(0), c.Da * logits.stride(2), logits.stride(1), logits.stride(2)),
       is = inits_strides(inits), gis = inits_strides(gi), hq(saved[6]), hk(saved[7]),
       hv(saved[8]), gq(g[0]), gk(g[1]), gv(g[2]);
   const Strides gvs(c.T * Fp, D, Fp, 1), gls(c.T * Fp, c.Da, Fp, 1);

@@ -95,6 +95,22 @@ def test_saved_tensor_hooks_streams_and_threads():
         _same(results[n], want, f"thread {n}")
 
 
+def test_saved_tensors_in_another_layout():
+    """Hooks may hand tensors back with the same values and other strides: x is
+    made contiguous and the scan reads any strides, as from Python."""
+    hm = _hm()
+    tensors, gs, dims = _case(3, 70, False, torch.bfloat16)
+
+    def other_layout(t):
+        return t.transpose(0, -1).contiguous().transpose(0, -1) if t.dim() > 2 else t
+
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, other_layout):
+        want = _step(hm._QkvFilterEager.apply, tensors, gs, dims)
+        _same(_step(hm.qkv_filter_call, tensors, gs, dims), want, "restrided")
+    for a, b in zip(want, _step(hm._QkvFilterEager.apply, tensors, gs, dims)):
+        assert float((a.double() - b.double()).norm()) <= 2.0 ** -7 * float(b.double().norm())
+
+
 def test_inputs_left_to_python():
     """Refused by the native entry, so that Python's own checks and paths apply."""
     hm = _hm()
