@@ -3,7 +3,7 @@
     python bench.py [--gpus 1] [--steps K] [--warmup W]
                     [--workload filter|look_back|gpt|scan_fwd|prefill|decode|peaks|lt_f32]
 
-Workload (BASELINE.json configs[2], the d12 training shape): x bf16
+Workload (the d12 training shape): x bf16
 [32, 1024, 768] ~ N(0, 1); c.weight [2322, 768] fp32 ~ N(0, 1/768) (value rows
 and the 18 gate rows, r = 128); logit_bias = 0; init_param ~ N(0, 1/768);
 upstream dq, dk, dv ~ N(0, 1).  Synthetic data, random-init weights.
@@ -16,25 +16,26 @@ in HBM before the timed region.  ``value`` = tokens / s = B*T*K / elapsed.
 Before the W warm-up steps, untimed steps of the same workload run for
 ``--settle-s`` seconds (0.1 by default; reported as ``settle``): after an idle
 period the GPU's clock ramps up over the first 15-20 ms of load (measured on
-MI355X at configs[2]: per-step times fall from 590-630 us to about 520 us over
+MI355X at this shape: per-step times fall from 590-630 us to about 520 us over
 the first ~30 steps of a process), and the metric is the steady-state rate of a
 training loop.  The timed region is still exactly K full steps.
 
 ``--workload look_back`` runs the same shapes through the look-back filter
 with the d12 layer spec (P, Q, K) = (16, 16, 9): chunks of 16 steps, each
 restarted from the inits over an 8-step warm-up (the reference's production
-look-back configuration).  ``--workload gpt`` is BASELINE.json configs[3].
-``--workload scan_fwd`` is configs[1], the standalone scan forward: bf16 head-major
+look-back configuration).  ``--workload gpt`` is one training
+step of the 12-layer d12 GPT with the filter in every layer.
+``--workload scan_fwd`` is the standalone scan forward: bf16 head-major
 values [32, 3 x 6, 1024, 128] ~ N(0, 1) with a per-element decay (r = 1)
 a = sigmoid(z), z ~ N(2, 1), i.e. logit + bias = -z; fp32 state, bf16 out; a
 step is one scan launch and ``value`` is its algorithmic GB/s.  ``--workload
-prefill`` is configs[4]'s prefill: one forward of the filter at B = 8,
+prefill`` is the long-sequence prefill: one forward of the filter at B = 8,
 T = 8192 with long-memory decays (tokens / s).  ``--workload decode`` is
-configs[4]'s decode: 256 single-token steps at B = 64 through the KV-cache
+the decode: 256 single-token steps at B = 64 through the KV-cache
 protocol after a 16-token prefill (tokens / s through the module), and the same
 256 steps replayed from a captured HIP graph.  ``--workload lt_f32`` is the
 filter's fp32 path's projection (the reference-layout ``fused_linear_transpose``,
-forward and both gradients) at configs[2]'s shapes, in TFLOP/s.
+forward and both gradients) at the d12 training shapes, in TFLOP/s.
 
 Printed as one JSON line, with
   roofline     -- the dominant kernel's algorithmic bytes (or FLOPs) per launch
@@ -235,18 +236,18 @@ def main():
                     choices=("filter", "look_back", "gpt", "scan_fwd", "prefill", "decode",
                              "peaks", "lt_f32"),
                     default="filter",
-                    help="filter: BASELINE.json configs[2] (the default, the metric's workload); "
+                    help="filter: the d12 training shape (the default, the metric's workload); "
                          "look_back: the same shapes through the look-back filter with the d12 "
                          "layer spec (16, 16, 9); "
-                         "gpt: configs[3], one training step of the 12-layer d12 GPT with the "
+                         "gpt: one training step of the 12-layer d12 GPT with the "
                          "filter in every layer (tokens/s and the filter's share of the step); "
-                         "scan_fwd: configs[1], the standalone per-element-decay scan forward "
-                         "(GB/s); prefill: configs[4]'s prefill, the filter forward at B=8, "
+                         "scan_fwd: the standalone per-element-decay scan forward "
+                         "(GB/s); prefill: the filter forward at B=8, "
                          "T=8192 with decay sigmoid(N(3, 1.5)) (tokens/s); "
                          "peaks: the measured roofline peaks (MFMA loop, HBM streams in the "
                          "scan's access shape, the library GEMM on the projection's shapes); "
                          "lt_f32: the filter's fp32 path's projection, fused_linear_transpose "
-                         "forward + backward at configs[2]'s shapes (TFLOP/s)")
+                         "forward + backward at the d12 training shapes (TFLOP/s)")
     ap.add_argument("--calibrate-copy", action="store_true",
                     help="after the timed region, run a plain device copy of 256 MiB five times "
                          "(the known-size reference for rocprofv3 FETCH_SIZE / WRITE_SIZE)")
@@ -420,11 +421,11 @@ def main():
     emit(out)
 
 
-# the standalone scan forward, per-element decay
+# The standalone scan forward, per-element decay
 SF_B, SF_H, SF_T, SF_D = 32, 18, 1024, 128
 
 
-# configs[1]'s and the d12 scan's arrays: 1,152 (b, head, 64-channel slab)
+# The standalone scan's and the d12 scan's arrays: 1,152 (b, head, 64-channel slab)
 # sequences of T = 1024 steps x 128 bytes, 151 MB per array
 PEAK_SLICES = 1152
 PEAK_SLICE_BYTES = 1024 * 128
@@ -554,7 +555,7 @@ def peaks_main(args):
 def lt_f32_main(args):
     """The filter's fp32 path projects through the reference-layout op
     ``fused_linear_transpose`` (x (B, T, C) . W (F, C)^T -> (B, F, T)).  One
-    step at configs[2]'s shapes is its forward and both gradients from a
+    step at the d12 training shapes is its forward and both gradients from a
     (B, F, T) grad_out, through the ops the fp32 filter's autograd calls (the
     backward with its split workspace); value is the step's TFLOP/s (3 GEMMs
     of 2 B T C F FLOP), the roofline the forward GEMM against a sixth
@@ -687,7 +688,7 @@ def lt_f32_cpu_baseline(seconds_target: float):
 
 
 def scan_fwd_bytes():
-    """Algorithmic bytes of one configs[1] launch: read the values and the
+    """Algorithmic bytes of one scan_fwd launch: read the values and the
     per-element logits, write the outputs (bf16), read the inits (bf16) and the
     fp32 bias (formula of the scan forward with Da = D, r = 1)."""
     n = SF_B * SF_H * SF_T * SF_D
@@ -695,7 +696,7 @@ def scan_fwd_bytes():
 
 
 def scan_fwd_cpu_baseline(seconds_target: float):
-    """The oracle's scan forward on one batch row of configs[1] (fp32 numpy)."""
+    """The oracle's scan forward on one batch row of scan_fwd (fp32 numpy)."""
     import numpy as np
     from threadpoolctl import threadpool_limits
 
@@ -726,7 +727,7 @@ def scan_fwd_cpu_baseline(seconds_target: float):
 
 
 def scan_fwd_main(args):
-    """one launch of the scan forward over bf16 head-major values
+    """One launch of the scan forward over bf16 head-major values
     (B, 18, T, D) with head-major per-element logits (B, 18, T, D) = -z."""
     import torch
     from nanochat_amd import _native as N
@@ -800,12 +801,12 @@ def scan_fwd_main(args):
     emit(out)
 
 
-# long-sequence prefill
+# Long-sequence prefill
 PF_B, PF_T = 8, 8192
 
 
 def prefill_main(args):
-    """configs[4]'s prefill: one forward of the drop-in filter (pack, bf16 MFMA
+    """The prefill: one forward of the drop-in filter (pack, bf16 MFMA
     projection, scan) on x bf16 [8, 8192, 768] ~ N(0, 1), c.weight ~
     N(0, 1/768) with the 18 gate rows scaled by 1.5 and logit_bias = -3, so
     logit + bias ~ N(-3, 1.5) and the decay a = sigmoid(z), z ~ N(3, 1.5), sits
@@ -901,12 +902,12 @@ def prefill_main(args):
     emit(out)
 
 
-# decode
+# Decode
 DC_B, DC_T0, DC_N = 64, 16, 256
 
 
 def decode_main(args):
-    """configs[4]'s decode: B = 64 sequences, a 16-token prefill, then 256
+    """The decode: B = 64 sequences, a 16-token prefill, then 256
     single-token steps through LtvCombinedQkvComputerModule and a KVCache (the
     filter state carried in the cache's last q/k/v rows).  A step is one token
     for the whole batch; ``--steps`` counts passes over the 256 tokens.
@@ -1031,7 +1032,7 @@ def decode_main(args):
 
 
 def gpt_main(args):
-    """one training step (forward + backward, no optimizer) of the
+    """One training step (forward + backward, no optimizer) of the
     12-layer d12 GPT on B=16, T=1024 token ids ~ U[0, 65536), random-init weights,
     bf16 autocast.  The filter's share is the summed duration of its library
     calls (HIP events on the launch stream) over the step time."""

@@ -504,12 +504,12 @@ int check_pqk(int P, int Q, int K) {
 // and it is chosen where the tile kernel would run fewer than 1,024
 // workgroups and each sequence spans at least 8 chunks (long T at small
 // batch).  Measured on MI355X:
-//   configs[4] prefill (B = 8, T = 8192, 288 sequences): tile 172 us, chained
+//   prefill (B = 8, T = 8192, 288 sequences): tile 172 us, chained
 //     (8, 8, 8) 127 us, (8, 16, 4) 128 us, (8, 8, 4) 145 us, (8, 4, 8) 135 us;
 //   d12 (1,152 sequences, T = 1024): tile 62.6 us, chained (8, 8, 8) 66.6 us,
 //     (8, 16, 4) 70.4 us -- with every sequence's workgroup resident the tile
 //     kernel streams without per-chunk start-up;
-//   configs[1] (r = 1, 1,152 sequences): tile 99.6 us, chained (8, 8, 4)
+//   per-channel gates (r = 1, 1,152 sequences): tile 99.6 us, chained (8, 8, 4)
 //     96.5 us, (8, 4, 4) 128 us.
 // Chunks shorter than 256 steps lose to the per-workgroup start-up (ticket,
 // two barriers, the hand-off): (8, 4, 4) 124 us, (8, 2, 4) 222 us at d12.

@@ -314,7 +314,7 @@ __device__ __forceinline__ Rsrc make_rsrc(const void* base) {
 }
 // Store cache policy (the instruction's aux bits): kStNormal, or kStStream
 // (gfx950 `nt`: non-temporal).  Measured on MI355X: streaming stores take the
-// per-channel-gate forward (r = 1, configs[1]) from 106 to 91 us; they slow the
+// per-channel-gate forward (r = 1) from 106 to 91 us; they slow the
 // d12 forward (62 -> 69 us) and the d12 backward (124 -> 128 us with streaming
 // value gradients, 168 us with streaming 2-byte logit gradients: partial-line
 // streaming writes), so everything else stores normally.
@@ -324,7 +324,7 @@ constexpr int kStStream = 2;
 // Measured on MI355X at d12: the backward's value, output-gradient and state
 // loads as streaming take it from 125 to 117 us, and the grad_x GEMM that
 // follows it from 135 to 122 us (the grad_combined it reads stays cached);
-// the forwards lose with them (configs[1] 95 -> 104 us, the look-back
+// the forwards lose with them (per-channel 95 -> 104 us, the look-back
 // window kernels 67 -> 72 and 176 -> 179 us), so only the tile backward
 // streams its loads.
 constexpr int kLdNormal = 0;
